@@ -209,6 +209,7 @@ struct SplitPlan {
     int schedule;     // PKV_SCHED_* (0 = invalid request)
     int splits;       // split slots per (b, h) row; the worker count for PKV_SCHED_TILES
     int split_tokens; // PKV_SCHED_WINDOWS: tokens per window
+    int prefill;      // > 0: PKV_SCHED_TILES through the prefill kernel, with this many workgroups
 };
 
 int64_t effective_max_seqlen(const pkv_decode_desc* d, const Resolved& r) {
@@ -292,6 +293,52 @@ bool single_pass_wins(const Resolved& r, int64_t max_seqlen, int workers) {
 }
 
 SplitPlan resolve_splits(const pkv_decode_desc* d, const Resolved& r, int num_splits);
+size_t workspace_bytes(const Resolved& r, const SplitPlan& plan);
+
+// Calls that the prefill kernel takes (pkv_prefill.hip) are those with enough
+// work for the matrix cores to matter: `work` counts 32-row x 64-token blocks,
+// bounded from max_seqlen.  Measured on MI355X (bf16, append and attention,
+// prefill / decode kernels, us): head_dim 128, work 4,128 (1 row of 32 query
+// tokens over 8,192, 32/8 heads) 38.6 / 34.9, 8,256 (64 tokens) 46.7 / 51.9,
+// 16,640 52.9 / 76.5, 270,336 (8 rows of 256 tokens) 421 / 973; head_dim 64,
+// 8,256 39.9 / 38.8, 16,640 47 / 57.5; head_dim 256, 8,256 77 / 69, 10,240 81 /
+// 94, 16,640 90 / 115.  Short rows of the same work gain earlier (4,480: 8 rows
+// of 1,792 query rows 40.5 / 47.9).  With 64 query rows per KV head half of
+// each row block would be empty (work 16,512: 82-90 / 85).
+constexpr int64_t kPrefillMinWork = 8192;
+constexpr int64_t kPrefillMinWorkD256 = 10240;
+constexpr int64_t kPrefillMinRows = 65;
+
+// Units (tiles and their streams' start) of a workgroup's share in a call that
+// does not fill the chip.  More workgroups cut the streams into more parts:
+// 1 row of 64 query tokens over 8,192 with 4 / 8 units: 63.4 / 48.2 us.
+constexpr int64_t kPrefillShare = 8;
+
+// Workgroups of the prefill kernel for this call; 0 = the decode kernels.  Two
+// per CU, one at head_dim 256 (128 KB of LDS).  Beside the work, the kernel's
+// own limits: pages that hold the token rows one load takes, page offsets of 32
+// bits, a plan that fits the LDS and 32-bit units.
+int prefill_groups(const pkv_decode_desc* d, const Resolved& r, int num_splits) {
+    if (num_splits != 0 || d->split_tokens != 0 || r.path != PKV_PATH_MFMA || r.rows < kPrefillMinRows || r.P < 8 ||
+        r.P * r.Hk * r.D * (r.kv_fp8 ? 1 : 2) >= (int64_t{1} << 32)) {
+        return 0;
+    }
+    const int64_t blocks = (r.rows + pkv::kPrefillRows - 1) / pkv::kPrefillRows;
+    const int64_t tiles = (row_tiles_bound(r, effective_max_seqlen(d, r)) + 3) / 4; // of 64 tokens
+    const int64_t work = r.B * r.Hk * ((r.rows + 31) / 32) * tiles;
+    if (work < (r.D == 256 ? kPrefillMinWorkD256 : kPrefillMinWork) || r.B * blocks > pkv::kPrefillEntries) {
+        return 0;
+    }
+    // Rows may be longer than max_seqlen: the 32-bit limits are for whole block-table rows.
+    const int64_t row_cap = d->block_table_stride * r.P;
+    const int64_t most_units = r.B * r.Hk * blocks * (row_cap / 64 + pkv::kPrefillHeader + 2);
+    if (row_cap > (int64_t{1} << 30) || most_units >= (int64_t{1} << 31)) {
+        return 0;
+    }
+    const int64_t units = r.B * r.Hk * blocks * (tiles + pkv::kPrefillHeader + 1);
+    const int64_t most = kComputeUnits * (r.D == 256 ? 1 : 2);
+    return static_cast<int>(std::clamp<int64_t>((units + kPrefillShare - 1) / kPrefillShare, 1, most));
+}
 
 // Paired KV heads make a wave's share half as many (twice as wide) units, so
 // each segment's start-up (page window, first tile) weighs twice as much.
@@ -301,11 +348,22 @@ SplitPlan resolve_splits(const pkv_decode_desc* d, const Resolved& r, int num_sp
 // 109.0 / 117.1, C4 (513) 127.4 / 130.0, C2 (32) 33.2 / 32.1.
 constexpr int64_t kPairMinShare = 64;
 
-// The plan of a call: resolve_splits, with KV heads paired (r updated) when
-// pairs_ok and the paired plan is the tile schedule with long shares; the
-// single pass, split schedules and the folded append stream one KV head per
-// wave.
-SplitPlan plan_call(const pkv_decode_desc* d, Resolved& r, int num_splits, bool fold) {
+// The plan of a call: the prefill kernel where it applies and its partials fit
+// the `workspace` bytes at hand (a caller whose workspace fits only the decode
+// kernels' plan keeps that one); else resolve_splits, with KV heads paired (r
+// updated) when pairs_ok and the paired plan is the tile schedule with long
+// shares; the single pass, split schedules and the folded append stream one KV
+// head per wave.
+SplitPlan plan_call(const pkv_decode_desc* d, Resolved& r, int num_splits, bool fold,
+                    size_t workspace = SIZE_MAX) {
+    if (!fold) {
+        const int groups = prefill_groups(d, r, num_splits);
+        const SplitPlan plan{PKV_SCHED_TILES, groups * pkv::kTileWaves, 0, groups};
+        if (groups > 0 && workspace_bytes(r, plan) <= workspace) {
+            r.head_groups = static_cast<int>((r.rows + pkv::kPrefillRows - 1) / pkv::kPrefillRows);
+            return plan;
+        }
+    }
     if (!fold && pairs_ok(r)) {
         const Resolved rp = paired(r);
         const SplitPlan pp = resolve_splits(d, rp, num_splits);
@@ -322,16 +380,16 @@ SplitPlan plan_call(const pkv_decode_desc* d, Resolved& r, int num_splits, bool 
 
 SplitPlan resolve_splits(const pkv_decode_desc* d, const Resolved& r, int num_splits) {
     if (num_splits < 0) {
-        return {0, 0, 0};
+        return {0, 0, 0, 0};
     }
     const int64_t max_seqlen = effective_max_seqlen(d, r);
     if (num_splits == 0) {
         if (d->split_tokens == 0) {
             const int workers = tile_workers(r, max_seqlen);
             if (single_pass_wins(r, max_seqlen, workers)) {
-                return {PKV_SCHED_SINGLE, 1, 0};
+                return {PKV_SCHED_SINGLE, 1, 0, 0};
             }
-            return {PKV_SCHED_TILES, workers, 0};
+            return {PKV_SCHED_TILES, workers, 0, 0};
         }
         int64_t tok = d->split_tokens;
         int64_t s = (max_seqlen + tok - 1) / tok;
@@ -340,14 +398,14 @@ SplitPlan resolve_splits(const pkv_decode_desc* d, const Resolved& r, int num_sp
             s = (max_seqlen + tok - 1) / tok;
         }
         if (s <= 1) {
-            return {PKV_SCHED_SINGLE, 1, 0};
+            return {PKV_SCHED_SINGLE, 1, 0, 0};
         }
-        return {PKV_SCHED_WINDOWS, static_cast<int>(s), static_cast<int>(tok)};
+        return {PKV_SCHED_WINDOWS, static_cast<int>(s), static_cast<int>(tok), 0};
     }
     int64_t s = std::min<int64_t>(num_splits, r.max_pages);
     s = std::min<int64_t>(s, PKV_MAX_SPLITS);
     s = std::max<int64_t>(1, s);
-    return {s == 1 ? PKV_SCHED_SINGLE : PKV_SCHED_PAGES, static_cast<int>(s), 0};
+    return {s == 1 ? PKV_SCHED_SINGLE : PKV_SCHED_PAGES, static_cast<int>(s), 0, 0};
 }
 
 constexpr size_t kAlign = 256;
@@ -357,6 +415,9 @@ size_t align_up(size_t x) { return (x + kAlign - 1) / kAlign * kAlign; }
 // Partial rows the plan stores: (b, h, split) rows for split schedules;
 // (workers + streams) slots of part_heads rows for the tile-balanced schedule.
 size_t partial_rows(const Resolved& r, const SplitPlan& plan) {
+    if (plan.prefill > 0) {
+        return static_cast<size_t>(plan.prefill) * 2 * pkv::kPrefillRows;
+    }
     if (plan.schedule == PKV_SCHED_TILES) {
         return static_cast<size_t>(plan.splits + r.B * streams_per_row(r)) * static_cast<size_t>(part_heads(r));
     }
@@ -371,7 +432,8 @@ size_t workspace_bytes(const Resolved& r, const SplitPlan& plan) {
     if (rows == 0) {
         return 0;
     }
-    return align_up(rows * static_cast<size_t>(r.D) * sizeof(float)) + align_up(rows * sizeof(float));
+    const size_t cuts = plan.prefill > 0 ? static_cast<size_t>(plan.prefill) * 4 * sizeof(int32_t) : 0;
+    return align_up(rows * static_cast<size_t>(r.D) * sizeof(float)) + align_up(rows * sizeof(float) + cuts);
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -482,7 +544,7 @@ constexpr int64_t kMaxFoldTokens = 8;
 // cached tokens; a cache_leftpad hides the same keys from every query, so the
 // partition applies it and the combine skips new tokens below it).
 bool fold_plan_ok(const Resolved& r, const pkv_decode_desc* d, const SplitPlan& plan) {
-    if (plan.schedule != PKV_SCHED_TILES || r.M > kMaxFoldTokens || r.win_left >= 0 || r.win_right >= 0 ||
+    if (plan.schedule != PKV_SCHED_TILES || plan.prefill > 0 || r.M > kMaxFoldTokens || r.win_left >= 0 || r.win_right >= 0 ||
         d->alibi_slopes != nullptr || d->softcap > 0.f || r.rotary) {
         return false;
     }
@@ -513,7 +575,8 @@ int decode_impl(const void* q, const void* k_cache, const void* v_cache, const i
     if (num_splits < 0 || !std::isfinite(softmax_scale)) {
         return PKV_EINVAL;
     }
-    const SplitPlan plan = plan_call(desc, r, num_splits, fold != nullptr);
+    const SplitPlan plan =
+        plan_call(desc, r, num_splits, fold != nullptr, desc->workspace != nullptr ? desc->workspace_bytes : 0);
     const bool tiles = plan.schedule == PKV_SCHED_TILES;
     const int splits = tiles ? 0 : plan.splits;
     const size_t need = workspace_bytes(r, plan);
@@ -594,6 +657,13 @@ int decode_impl(const void* q, const void* k_cache, const void* v_cache, const i
         comb_ev = {ev[2], ev[3]};
     }
 
+    if (plan.prefill > 0) {
+        p.tile_workers = plan.prefill;
+        if (pkv::launch_prefill(p, bf16, static_cast<int>(r.D), s, part_ev, comb_ev) != hipSuccess) {
+            return PKV_ELAUNCH;
+        }
+        return PKV_OK;
+    }
     const hipError_t e = pkv::launch_partition(p, r.path == PKV_PATH_MFMA, bf16, static_cast<int>(r.D),
                                                r.heads_per_wave, s, part_ev);
     if (e != hipSuccess) {
@@ -811,7 +881,8 @@ int pkv_decode_noalloc(const void* q, const void* k_cache, const void* v_cache, 
     if (st != PKV_OK) {
         return st;
     }
-    if (num_splits >= 0 && workspace_bytes(r, plan_call(desc, r, num_splits, false)) > PKV_SCRATCH_BYTES) {
+    if (num_splits >= 0 &&
+        workspace_bytes(r, plan_call(desc, r, num_splits, false, PKV_SCRATCH_BYTES)) > PKV_SCRATCH_BYTES) {
         return PKV_ENOWORKSPACE;
     }
     void* ptr = nullptr;

@@ -126,6 +126,16 @@ struct FoldParams {
 // Query rows per wave of the tile schedule's stream combine.
 constexpr int kStreamRows = 4;
 
+// Query rows per workgroup of the prefill kernel (pkv_prefill.hip).
+constexpr int kPrefillRows = 128;
+// Row blocks of a call (batch rows x blocks) its plan holds in the LDS.
+constexpr int kPrefillEntries = 2048;
+// Units a stream is charged for its start (page ids, q, first tiles) and the
+// writing of its rows.  With 1 / 2 / 3 (and a snap of the same): 4 x 512 query
+// tokens over 0-4,096 145.7 / 140.5 / 140.9 us, 3 x 333 with a 1,024-token window
+// at head_dim 256 76.8 / 78.1 / 83.9, 2,048 tokens without a context 100 / 86 / 88.
+constexpr int kPrefillHeader = 2;
+
 // Paged KV-cache append (pkv_append.hip): one 16-byte chunk of K and of V per
 // thread.  A token row is Hk * D 16-bit elements, contiguous in the new-token
 // tensors ([tokens, Hk, D]) and in its cache slot ([num_pages, P, Hk, D]).

@@ -36,6 +36,12 @@ inline void launch_kernel(void (*kernel)(KArgs...), dim3 grid, dim3 block, size_
 hipError_t launch_partition(const PartitionParams& p, bool mfma, bool bf16, int head_dim, int heads_per_wave,
                             hipStream_t stream, const LaunchEvents& ev);
 
+// Many query rows per KV head (pkv_prefill.hip): p.tile_workers workgroups share
+// the call's tiles, p.head_groups row blocks of kPrefillRows per KV head; then
+// the merge of the streams they cut.
+hipError_t launch_prefill(const PartitionParams& p, bool bf16, int head_dim, hipStream_t stream,
+                          const LaunchEvents& part_ev, const LaunchEvents& comb_ev);
+
 // LSE combine of split partials into the 16-bit output; with `fold` (tile
 // schedule only) the combine also adds and stores the appended tokens.
 hipError_t launch_combine(const CombineParams& p, const FoldParams* fold, bool bf16, int head_dim,

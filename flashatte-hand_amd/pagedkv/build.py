@@ -28,7 +28,7 @@ TORCH_BINDING_SRC = PKG_ROOT / "binding" / "pkv_torch.cpp"
 ORACLE_DIR = REPO_ROOT / "oracle"
 ORACLE_LIB = ORACLE_DIR / "libpkv_oracle.so"
 
-SOURCES = ["pkv_part_d128.hip", "pkv_part_d256.hip", "pkv_part_d64.hip", "pkv_partition.hip",
+SOURCES = ["pkv_prefill.hip", "pkv_part_d128.hip", "pkv_part_d256.hip", "pkv_part_d64.hip", "pkv_partition.hip",
            "pkv_combine.hip", "pkv_append.hip", "pkv_api.cpp"]
 
 HIPCC_FLAGS = [

@@ -561,3 +561,37 @@ def test_head_groups_share_a_gang_on_the_tile_schedule():
         assert pagedkv.schedule_for(d, 0) == pagedkv.PKV_SCHED_TILES
         rows = (pagedkv.num_splits_for(d, 0) + 4 * 2) * 32  # (waves + B x 2 head groups) slots of 32 rows
         assert pagedkv.workspace_size(d, 0) == align(rows * 256 * 4) + align(rows * 4)
+
+
+@pytest.mark.parametrize("change,prefill", [
+    ({}, True),
+    ({"head_dim": 64}, True),
+    ({"kv_dtype": pagedkv.PKV_KV_DTYPE_FP8_E4M3}, True),
+    ({"seqlen_q": 16}, False),               # 64 query rows per KV head: half of every row block empty
+    ({"max_seqlen": 4095, "batch": 1}, False),  # 4,096 blocks of 32 rows x 64 tokens
+    ({"head_dim": 256, "batch": 1}, False),  # 8,192 blocks: enough at head_dim 128, not at 256
+    ({"batch": 1}, True),
+    ({"page_size": 4}, False),               # a load's token rows would span pages
+    ({"split_tokens": 512}, False),
+    ({"path": pagedkv.PKV_PATH_VALU, "seqlen_q": 1}, False),
+])
+def test_prefill_kernel_in_the_plan(change, prefill):
+    """Calls with more than 64 query rows per KV head and enough 32-row x 64-token blocks of work
+    (bounded from max_seqlen) plan the prefill kernel: the tile schedule with two partial slots of
+    128 rows and 16 bytes per workgroup, at most two workgroups per CU (one at head_dim 256)."""
+    align = lambda x: (x + 255) // 256 * 256  # noqa: E731
+    kw = dict(batch=4, num_heads=32, num_heads_k=8, head_dim=128, page_size=16, block_table_stride=512,
+              max_seqlen=8192, num_pages=4096, seqlen_q=64)
+    kw.update(change)
+    if kw["page_size"] == 4:
+        kw["block_table_stride"] = 2048
+    d = base_desc(**kw)
+    waves, need = pagedkv.num_splits_for(d, 0), pagedkv.workspace_size(d, 0)
+    rows = waves // 4 * 2 * 128
+    D = kw["head_dim"]
+    is_prefill = need == align(rows * D * 4) + align(rows * 4 + waves // 4 * 16)
+    assert is_prefill == prefill
+    if prefill:
+        assert pagedkv.schedule_for(d, 0) == pagedkv.PKV_SCHED_TILES
+        assert waves % 4 == 0 and waves // 4 <= 512
+    assert pagedkv.schedule_for(d, 3) in (0, pagedkv.PKV_SCHED_PAGES)  # forced splits never take it

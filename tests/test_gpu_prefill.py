@@ -1,0 +1,179 @@
+"""GPU parity of the prefill kernel (csrc/pkv_prefill.hip: many query rows per KV head) against the
+fp64 oracle, at the edges of its row blocks (128 rows, 32 per wave), tiles (64 tokens, blocks of
+32) and shares: rows and lengths on both sides of each, empty and very short rows, streams cut
+into many parts and streams that fit one share, every head_dim and cache type, each mask, and
+NaN bytes everywhere no query sees.
+
+The library takes the kernel for calls with enough work, judged from the block table's width; the
+cases here widen the table instead of the rows, and check that the call's plan is the prefill
+kernel's (its workspace is 2 partial slots of 128 rows per workgroup).  Tolerances are the
+decode's (test_gpu_fp8.assert_close): the kernel carries the same precision.
+"""
+from __future__ import annotations
+
+import math
+
+import numpy as np
+import pytest
+
+import pkv_oracle as po
+from conftest import gpu_available, make_case, rand_bits
+from test_gpu_fp8 import assert_close, f32, fp8_cache, i32, to_dev8
+from test_gpu_lse import assert_lse, lse_buffer
+from test_gpu_parity import announce, to_dev, torch_mod
+
+pytestmark = [pytest.mark.gpu, pytest.mark.skipif(not gpu_available(), reason="needs a GPU")]
+
+# H, Hk, D, P, lens, M, options
+CASES = [
+    (8, 2, 128, 16, [700, 130, 129, 1], 33, dict(causal=True)),
+    (28, 4, 128, 64, [64, 65, 1000], 37, dict(causal=True, dtype=0)),          # group 7: rows end inside a block
+    (4, 4, 128, 8, [257, 300], 129, dict(causal=True)),                        # one query row past a block
+    (16, 1, 128, 256, [2100], 16, dict(causal=False)),                         # one stream pair, many parts
+    (8, 2, 128, 32, [40, 20, 0], 64, dict(causal=True)),                       # more queries than keys
+    (8, 2, 128, 16, [900, 500], 64, dict(causal=True, window=(300, 0), alibi=True)),
+    (8, 2, 128, 16, [900, 31], 40, dict(causal=False, window=(400, 5), softcap=20.0)),
+    (8, 2, 128, 16, [600, 333], 40, dict(causal=True, leftpad=[95, 333])),
+    (8, 2, 128, 64, [600, 95], 40, dict(causal=True, fp8=True)),
+    (8, 2, 128, 64, [600, 95], 40, dict(causal=True, fp8=True, dtype=0, leftpad=[33, 0], scale=-0.1)),
+    (8, 8, 64, 16, [95, 96, 97, 640], 70, dict(causal=True)),
+    (8, 2, 64, 8, [700, 31], 40, dict(causal=True, fp8=True, alibi=True)),
+    (8, 2, 256, 16, [700, 33, 1], 40, dict(causal=True, dtype=0)),
+    (4, 2, 256, 32, [400, 320], 100, dict(causal=True, window=(390, 0), softcap=30.0)),
+    (8, 2, 256, 64, [300, 65], 40, dict(causal=True, fp8=True)),
+]
+
+
+def desc_plan(q, kc, bt, **kw):
+    """(waves, workspace bytes) of the call's plan."""
+    import pagedkv
+
+    B, M, H, D = q.shape
+    d = pagedkv.make_desc(batch=B, num_heads=H, num_heads_k=kc.shape[2], head_dim=D, page_size=kc.shape[1],
+                          num_pages=kc.shape[0], block_table_stride=bt.shape[1], seqlen_q=M, **kw)
+    return pagedkv.num_splits_for(d), pagedkv.workspace_size(d)
+
+
+def prefill_workspace(waves, D):
+    assert waves > 0
+    rows = waves // 4 * 2 * 128
+    up = lambda x: (x + 255) // 256 * 256  # noqa: E731
+    return up(rows * D * 4) + up(rows * 4 + waves // 4 * 16)
+
+
+def hide(kc, vc, bt, lens, leftpad, nan):
+    """Fill every slot that no query sees with `nan`."""
+    P = kc.shape[1]
+    seen = np.zeros(kc.shape[:2], bool)
+    for b, n in enumerate(lens):
+        t = np.arange(0 if leftpad is None else leftpad[b], max(n, 0))
+        seen[bt[b, t // P], t % P] = True
+    kc[~seen] = nan
+    vc[~seen] = nan
+
+
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_prefill_matches_oracle(case):
+    import pagedkv
+
+    torch = torch_mod()
+    H, Hk, D, P, lens, M, opt = CASES[case]
+    announce("prefill", CASES[case])
+    rng = np.random.default_rng(9100 + case)
+    dtype, fp8, B = opt.get("dtype", 1), opt.get("fp8", False), len(lens)
+    window, leftpad = opt.get("window", (-1, -1)), opt.get("leftpad")
+    blocks = B * Hk * -(-(M * H // Hk) // 32)
+    stride = -(-12000 * 64 // blocks) // P + 1  # a table wide enough for the kernel to be chosen
+    if window[0] >= 0:
+        H, Hk, lens, B = H * 8, Hk * 8, lens * 8, B * 8  # a window bounds the work: more rows instead
+        leftpad = None if leftpad is None else leftpad * 8
+        stride = 1
+    _, kc, vc, bt, sl = make_case(rng, B=B, H=H, Hk=Hk, D=D, P=P, seqlens=lens, dtype=dtype, stride=stride)
+    q = rand_bits(rng, (B, M, H, D), dtype)
+    scale = opt.get("scale", 1.0 / math.sqrt(D))
+    slopes = rng.uniform(0.01, 0.3, size=(B, H)).astype(np.float32) if opt.get("alibi") else None
+    cap = opt.get("softcap", 0.0)
+    ks = vs = None
+    kw = dict(causal=opt["causal"], window=window, alibi=slopes, lse=True, leftpad=None if leftpad is None else
+              np.asarray(leftpad, np.int32), softcap=cap)
+    if fp8:
+        ks, vs = (rng.uniform(0.2, 2.0, Hk).astype(np.float32) for _ in range(2))
+        kc, vc = fp8_cache(rng, kc.shape, ks), fp8_cache(rng, vc.shape, vs)
+        want, want_lse = po.attn8_f64(q, kc, vc, bt, sl, scale, dtype, k_scale=ks, v_scale=vs, **kw)
+        hide(kc, vc, bt, lens, leftpad, 0x7F)
+        kd, vd = to_dev8(kc), to_dev8(vc)
+    else:
+        want, want_lse = po.attn_f64(q, kc, vc, bt, sl, scale, dtype, **kw)
+        hide(kc, vc, bt, lens, leftpad, 0x7FC0 if dtype == 1 else 0x7E00)
+        kd, vd = to_dev(kc, dtype), to_dev(vc, dtype)
+    waves, need = desc_plan(q, kc, bt, dtype=dtype, causal=opt["causal"], window_size=window,
+                            kv_dtype=pagedkv.PKV_KV_DTYPE_FP8_E4M3 if fp8 else 0)
+    assert need == prefill_workspace(waves, D)
+    lse = lse_buffer(B, H, M)
+    args = (to_dev(q, dtype), kd, vd, i32(bt), i32(sl), scale, 0)
+    more = dict(causal=opt["causal"], window_size=window, alibi_slopes=f32(slopes), k_scale=f32(ks), v_scale=f32(vs),
+                softcap=cap, cache_leftpad=None if leftpad is None else i32(np.asarray(leftpad, np.int32)))
+    out = pagedkv.decode(*args, softmax_lse=lse, **more)
+    torch.cuda.synchronize()
+    assert_close(out, want, dtype)
+    assert_lse(lse, want_lse)
+    # A workspace that only the decode kernels' plan fits (1,024 waves' and the streams' slots of 32
+    # rows at most): that plan, within the same tolerance.
+    if need - 256 >= (1024 + B * Hk * -(-(M * H // Hk) // 32)) * 32 * (D + 1) * 4 + 512:
+        small = pagedkv.decode(*args, workspace=torch.empty(need - 256, dtype=torch.uint8, device="cuda"), **more)
+        torch.cuda.synchronize()
+        assert_close(small, want, dtype)
+
+
+def test_prefill_many_ragged_rows():
+    """More rows than threads in a workgroup, one to three row blocks each, rows without tokens
+    among them: shares cross rows, blocks and KV heads."""
+    import pagedkv
+
+    torch = torch_mod()
+    announce("prefill-ragged")
+    rng = np.random.default_rng(9200)
+    B, H, Hk, D, P, M, dtype = 300, 4, 2, 128, 16, 70, 1
+    lens = rng.integers(0, 400, size=B).astype(np.int32)
+    lens[:3] = (0, 1, 399)
+    _, kc, vc, bt, sl = make_case(rng, B=B, H=H, Hk=Hk, D=D, P=P, seqlens=lens, dtype=dtype)
+    q = rand_bits(rng, (B, M, H, D), dtype)
+    want = po.attn_f64(q, kc, vc, bt, sl, 0.09, dtype, causal=True)
+    waves, need = desc_plan(q, kc, bt, dtype=dtype, causal=True)
+    assert need == prefill_workspace(waves, D)
+    out = pagedkv.decode(to_dev(q, dtype), to_dev(kc, dtype), to_dev(vc, dtype), i32(bt), i32(sl), 0.09, 0,
+                         causal=True)
+    torch.cuda.synchronize()
+    assert_close(out, want, dtype)
+
+
+def test_prefill_under_graph_replays():
+    """A captured appending prefill chunk, replayed several times with eager work in between."""
+    import pagedkv
+
+    torch = torch_mod()
+    announce("prefill-graph")
+    rng = np.random.default_rng(9300)
+    B, H, Hk, D, P, M, dtype = 2, 32, 8, 128, 16, 96, 1
+    _, kc, vc, bt, sl = make_case(rng, B=B, H=H, Hk=Hk, D=D, P=P, seqlens=[1500, 700], dtype=dtype)
+    q, kd, vd = to_dev(rand_bits(rng, (B, M, H, D), dtype), dtype), to_dev(kc, dtype), to_dev(vc, dtype)
+    kn, vn = (to_dev(rand_bits(rng, (B, M, Hk, D), dtype), dtype) for _ in range(2))
+    table, lens = i32(bt), i32(np.asarray(sl) - M)
+
+    def call():
+        return pagedkv.decode(q, kd, vd, table, lens, 0.09, 0, k_new=kn, v_new=vn, causal=True)
+
+    want = call().clone()
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        got = call()
+    for _ in range(4):
+        got.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+        assert torch.equal(call(), want)
