@@ -177,7 +177,7 @@ __device__ __forceinline__ void dma_wait() { asm volatile("s_waitcnt vmcnt(0)" :
 
 typedef __attribute__((address_space(3))) uint16_t lds_u16;
 
-template <bool BF16, int D, bool FP8>
+template <bool BF16, int D, bool FP8, bool CAP>
 __global__ __launch_bounds__(kThreads, D == 256 ? 1 : 2) void prefill_kernel(PartitionParams p) {
     using C = Prefill<BF16, D, FP8>;
     constexpr int kTok = C::kTok;
@@ -452,7 +452,8 @@ __global__ __launch_bounds__(kThreads, D == 256 ? 1 : 2) void prefill_kernel(Par
             const float slope =
                 alibi ? p.alibi[static_cast<int64_t>(b) * p.alibi_stride + head] * 1.4426950408889634f : 0.f;
             const float cap = p.softcap_log2;
-            const float inv_cap = cap > 0.f ? 1.f / cap : 0.f;
+            const float inv_cap = CAP ? 1.f / cap : 0.f;
+            const float cap_rate = -2.8853900817779268f * scale * inv_cap; // -2 log2(e) scale / cap
 
             f32x16 o[C::DT];
 #pragma unroll
@@ -503,70 +504,43 @@ __global__ __launch_bounds__(kThreads, D == 256 ? 1 : 2) void prefill_kernel(Par
             const int vdim = ((lane & 16) ? C::kSplit : 0) + 4 * (lane & 3);
             uint32_t vaddr = smem_at + 2 * (vrow * D + 8 * ((vdim >> 3) ^ C::swz(vrow)) + (vdim & 7));
             const auto read_k = [&](int at, int kk) {
-                const u32x4 v = *(const lds_u32x4*)(uintptr_t)((kaddr ^ (32 * kk)) + 2 * at);
+                const u32x4 v = *(const lds_u32x4*)(uintptr_t)((kaddr ^ (32 * (kk & 7))) + 256 * (kk >> 3) + 2 * at);
                 return make_uint4(v.x, v.y, v.z, v.w);
             };
             // V^T of dims tile dt, tokens 16 u .. 16 u + 15 of the block: half e.
             const auto read_v4 = [&](int at, int u, int dt, int e) {
-                const uint32_t a = vaddr ^ (2 * C::dim0(dt) + (e ? C::kFlip8 : 0)); // half 1: eight rows on
+                // Half 1 is eight rows on; dims from 128 on are 256 bytes on (swz moves within those).
+                const uint32_t a = (vaddr ^ ((2 * C::dim0(dt) & 255) + (e ? C::kFlip8 : 0))) + (2 * C::dim0(dt) & ~255);
                 return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)(
                                                      a + 2 * (at + (16 * u + 8 * e) * D))));
             };
-            const bool special = alibi || cap > 0.f;
-
             f32x16 s[2];      // scores of an even / odd block
             uint4 ph[2][2];   // probabilities of an even / odd block: heads of its two 16-token steps
             uint4 pl[2][2];   // and their remainders
             float alpha = 1.f;
             bool raise = false;
 
-            // One block of the pipeline: the scores of the next block (K block
-            // `j` of the tile's buffers), the product of the last block's
-            // probabilities (V block `j`), and between them the softmax of
-            // this block, whose tokens start at t.
-            const auto block = [&](auto jc, auto bufc, int t) {
+            // The slots of one block (below).  `mul` takes the scores to log2 units.
+            // With a softcap raw scores are capped first (`done`: they are already):
+            // cap tanh(x / cap), tanh |y| = (1 - e) / (1 + e), e = exp(-2 |y|), times cap
+            // as `mul`.  (Capped outside the slots, 4 x 512 query tokens over 2,048 with a
+            // softcap took 137.7 / 175.3 us at head_dim 64 / 128, now 126.1 / 168.7;
+            // without one 94 / 138.)
+            const auto slots = [&](auto jc, auto bufc, bool done, float mul) {
                 constexpr int j = decltype(jc)::value;
                 constexpr int kat = decltype(bufc)::value * C::kBuf + j * 32 * D;
                 constexpr int vat = kat + 2 * C::kBuf;
                 f32x16& cur = s[j];
                 f32x16& next = s[j ^ 1];
-                float mul = scale;
-                if (special || t < all_lo || t + 32 > all_hi) {
-                    mul = 1.f;
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) {
-                        cur[i] *= scale;
-                    }
-                    if (cap > 0.f) {
-#pragma unroll
-                        for (int i = 0; i < 16; ++i) {
-                            cur[i] = cap * tanh_f32(cur[i] * inv_cap);
-                        }
-                    }
-                    if (alibi) {
-                        const float d = static_cast<float>(pos - t - 4 * h);
-#pragma unroll
-                        for (int i = 0; i < 16; ++i) {
-                            cur[i] -= slope * fabsf(d - static_cast<float>(8 * (i >> 2) + (i & 3)));
-                        }
-                    }
-                    if (t < all_lo || t + 32 > all_hi) {
-                        const int from = lo - t - 4 * h;
-                        const int upto = hi - t - 4 * h;
-#pragma unroll
-                        for (int i = 0; i < 16; ++i) {
-                            const int tok = 8 * (i >> 2) + (i & 3);
-                            cur[i] = tok >= from && tok < upto ? cur[i] : kNegInf;
-                        }
-                    }
-                }
                 // One basic block, in slots of one product each: what a slot
                 // holds beside it (an operand read kLead slots ahead, a load pass,
                 // a step of the softmax) issues while the products run.
                 asm volatile("" : "+v"(kaddr), "+v"(vaddr)); // operand addresses are made anew (kept, they spill)
                 constexpr int kSlots = C::KK + 4 * C::DT;
                 constexpr int kLead = 6;
-                constexpr int kSoftmax = kSlots >= 24 ? 5 : 2; // slots of the maximum; 16 half pairs of probabilities follow
+                constexpr int kCap = CAP ? kSlots / 3 >= 16 ? 16 : kSlots / 3 >= 8 ? 8 : 4 : 0; // slots of the cap,
+                constexpr int kSoftmax = kCap + (kSlots >= 24 ? 5 : 2); // of the maximum; 16 half pairs of
+                                                                        // probabilities follow
                 constexpr int kHalves = 16;
                 uint4 ka[C::KK];
                 uint2 va[4 * C::DT]; // halves of operand (u, dt)
@@ -612,13 +586,20 @@ __global__ __launch_bounds__(kThreads, D == 256 ? 1 : 2) void prefill_kernel(Par
                             load_pass(j * C::NP + pass, (1 - decltype(bufc)::value) * C::kBuf);
                         }
                     }
-                    if constexpr (i < kSoftmax) {
+                    if constexpr (i < kCap) {
+                        constexpr int kPer = 16 / (kCap > 0 ? kCap : 16);
+#pragma unroll
+                        for (int e = kPer * i; e < kPer * (i + 1); ++e) {
+                            const float y = fast_exp2(cap_rate * fabsf(cur[e]));
+                            cur[e] = done ? cur[e] : copysignf((1.f - y) * __builtin_amdgcn_rcpf(1.f + y), cur[e]);
+                        }
+                    } else if constexpr (i < kSoftmax) {
                         // The row maximum and what it changes.
-                        constexpr int kPer = 16 / (kSoftmax - 1);
+                        constexpr int kPer = 16 / (kSoftmax - kCap - 1);
                         if constexpr (i + 1 < kSoftmax) {
 #pragma unroll
                             for (int e = 0; e < kPer; ++e) {
-                                tmax = fmaxf(tmax, cur[kPer * i + e]);
+                                tmax = fmaxf(tmax, cur[kPer * (i - kCap) + e]);
                             }
                         } else {
                             tmax = max_halves32(tmax) * mul;
@@ -657,6 +638,46 @@ __global__ __launch_bounds__(kThreads, D == 256 ? 1 : 2) void prefill_kernel(Par
                     pl[j][u] = make_uint4(lp[4 * u], lp[4 * u + 1], lp[4 * u + 2], lp[4 * u + 3]);
                 }
                 l = fmaf(l, alpha, sum[0] + sum[1]);
+            };
+
+            // One block of the pipeline: the scores of the next block (K block
+            // `j` of the tile's buffers), the product of the last block's
+            // probabilities (V block `j`), and between them the softmax of
+            // this block, whose tokens start at t.
+            // A softcap's kernel caps the scores in the slots, except in blocks
+            // that also mask or bias them.
+            const auto block = [&](auto jc, auto bufc, int t) {
+                f32x16& cur = s[decltype(jc)::value];
+                const bool edge = alibi || t < all_lo || t + 32 > all_hi;
+                if (edge) {
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) {
+                        cur[i] *= scale;
+                    }
+                    if constexpr (CAP) {
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) {
+                            cur[i] = cap * tanh_f32(cur[i] * inv_cap);
+                        }
+                    }
+                    if (alibi) {
+                        const float d = static_cast<float>(pos - t - 4 * h);
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) {
+                            cur[i] -= slope * fabsf(d - static_cast<float>(8 * (i >> 2) + (i & 3)));
+                        }
+                    }
+                    if (t < all_lo || t + 32 > all_hi) {
+                        const int from = lo - t - 4 * h;
+                        const int upto = hi - t - 4 * h;
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) {
+                            const int tok = 8 * (i >> 2) + (i & 3);
+                            cur[i] = tok >= from && tok < upto ? cur[i] : kNegInf;
+                        }
+                    }
+                }
+                slots(jc, bufc, edge, edge ? 1.f : CAP ? cap : scale);
                 // O holds the products up to the last block's, relative to the old
                 // maximum.
                 if (__any(raise)) {
@@ -907,10 +928,18 @@ __global__ __launch_bounds__(16 * R) void prefill_combine_kernel(PartitionParams
 template <bool BF16, int D>
 hipError_t launch_d(const PartitionParams& p, hipStream_t stream, const LaunchEvents& part_ev,
                     const LaunchEvents& comb_ev) {
+    const dim3 grid(p.tile_workers);
+    const dim3 block(kThreads);
     if (p.kv_fp8) {
-        launch_kernel(prefill_kernel<BF16, D, true>, dim3(p.tile_workers), dim3(kThreads), 0, stream, part_ev, p);
+        if (p.softcap_log2 > 0.f) {
+            launch_kernel(prefill_kernel<BF16, D, true, true>, grid, block, 0, stream, part_ev, p);
+        } else {
+            launch_kernel(prefill_kernel<BF16, D, true, false>, grid, block, 0, stream, part_ev, p);
+        }
+    } else if (p.softcap_log2 > 0.f) {
+        launch_kernel(prefill_kernel<BF16, D, false, true>, grid, block, 0, stream, part_ev, p);
     } else {
-        launch_kernel(prefill_kernel<BF16, D, false>, dim3(p.tile_workers), dim3(kThreads), 0, stream, part_ev, p);
+        launch_kernel(prefill_kernel<BF16, D, false, false>, grid, block, 0, stream, part_ev, p);
     }
     // Few streams of many parts each need the workgroups; many cut streams fill
     // the chip as it is, and fewer workgroups are dispatched.
