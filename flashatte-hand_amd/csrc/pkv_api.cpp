@@ -314,6 +314,22 @@ constexpr int64_t kPrefillMinRows = 65;
 // 1 row of 64 query tokens over 8,192 with 4 / 8 units: 63.4 / 48.2 us.
 constexpr int64_t kPrefillShare = 8;
 
+// A verify step's append folds into the decode combine at no launch of its own,
+// so it leaves that path later.  Measured folded / append and prefill kernel (us,
+// 80-128 query rows per KV head): head_dim 64, work 12,000 37.5 / 41.4, 16,000 52.6 /
+// 40.5; head_dim 128, 12,000 (FP8) 50.5 / 52.0, 18,048 74.0 / 56.0; head_dim 256,
+// 12,096 158 / 91.
+constexpr int64_t kPrefillMinFoldWork = 12288;
+
+// 64-token tiles of a row, and the call's work, bounded from max_seqlen.
+int64_t prefill_tiles(const pkv_decode_desc* d, const Resolved& r) {
+    return (row_tiles_bound(r, effective_max_seqlen(d, r)) + 3) / 4;
+}
+
+int64_t prefill_work(const pkv_decode_desc* d, const Resolved& r) {
+    return r.B * r.Hk * ((r.rows + 31) / 32) * prefill_tiles(d, r);
+}
+
 // Workgroups of the prefill kernel for this call; 0 = the decode kernels.  Two
 // per CU, one at head_dim 256 (128 KB of LDS).  Beside the work, the kernel's
 // own limits: pages that hold the token rows one load takes, page offsets of 32
@@ -324,9 +340,9 @@ int prefill_groups(const pkv_decode_desc* d, const Resolved& r, int num_splits) 
         return 0;
     }
     const int64_t blocks = (r.rows + pkv::kPrefillRows - 1) / pkv::kPrefillRows;
-    const int64_t tiles = (row_tiles_bound(r, effective_max_seqlen(d, r)) + 3) / 4; // of 64 tokens
-    const int64_t work = r.B * r.Hk * ((r.rows + 31) / 32) * tiles;
-    if (work < (r.D == 256 ? kPrefillMinWorkD256 : kPrefillMinWork) || r.B * blocks > pkv::kPrefillEntries) {
+    const int64_t tiles = prefill_tiles(d, r);
+    if (prefill_work(d, r) < (r.D == 256 ? kPrefillMinWorkD256 : kPrefillMinWork) ||
+        r.B * blocks > pkv::kPrefillEntries) {
         return 0;
     }
     // Rows may be longer than max_seqlen: the 32-bit limits are for whole block-table rows.
@@ -788,10 +804,14 @@ pkv_decode_desc appended_desc(const pkv_decode_desc* d, int64_t seqlen_new) {
 // partition attends the cached tokens with `*part` = the appended-length
 // descriptor `a` without its causal mask (every query sits past them), the
 // combine adds the new tokens each query sees and stores them, and no append
-// kernel runs.  Other calls append first and then attend the longer rows.
+// kernel runs.  Other calls append first and then attend the longer rows, and so
+// do steps of more than 64 query rows per KV head with the prefill kernel's work.
 bool fold_fits(const pkv_decode_desc* a, int num_splits, int64_t seqlen_new, pkv_decode_desc* part, bool* causal) {
     Resolved r;
     if (resolve(a, r) != PKV_OK || seqlen_new != r.M || r.rotary) {
+        return false;
+    }
+    if (prefill_groups(a, r, num_splits) > 0 && (r.D == 256 || prefill_work(a, r) >= kPrefillMinFoldWork)) {
         return false;
     }
     *part = *a;

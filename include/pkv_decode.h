@@ -152,7 +152,10 @@ typedef struct pkv_decode_desc {
  *       all rows' 16-token tiles (times KV heads and head groups) are laid end
  *       to end and dealt in equal shares to one workgroup of waves per CU,
  *       which read cache_seqlens on the device, so every wave streams the same
- *       bytes however ragged the rows are, and a combine merges the rows that
+ *       bytes however ragged the rows are (calls with more than 64 query rows
+ *       per KV head and enough work: 64-token tiles dealt to workgroups that
+ *       share each tile; a workspace that only the waves' partials fit keeps
+ *       the waves), and a combine merges the rows that
  *       more than one wave touched.  Calls too small to fill the chip
  *       (rows of a few tiles, judged from max_seqlen), and calls whose left
  *       window bounds every row, take the single pass instead when its
@@ -296,7 +299,8 @@ size_t pkv_decode_append_workspace_size(const pkv_decode_desc* desc, int num_spl
  * is invalid.  Folded: as many new tokens as query tokens, at most 8 (the
  * decode step and the speculative verify step, causal or not), 16-bit or
  * FP8 caches, no window, ALiBi, softcap or rotary tables, the tile schedule
- * with its row-per-wave combine.  The outputs agree within the decode
+ * with its row-per-wave combine, and not so many query rows per KV head (over
+ * 64) and tokens that the kernel for prefill chunks is the faster one.  The outputs agree within the decode
  * tolerances (the new tokens' scores are summed in a different order); the
  * caches are written identically.  No
  * counterpart in the reference, whose decode never appends

@@ -595,3 +595,15 @@ def test_prefill_kernel_in_the_plan(change, prefill):
         assert pagedkv.schedule_for(d, 0) == pagedkv.PKV_SCHED_TILES
         assert waves % 4 == 0 and waves // 4 <= 512
     assert pagedkv.schedule_for(d, 3) in (0, pagedkv.PKV_SCHED_PAGES)  # forced splits never take it
+
+
+@pytest.mark.parametrize("max_seqlen,D,folds", [(3000, 128, True), (5000, 128, False), (3600, 64, True),
+                                                (3600, 256, False)])
+def test_long_verify_steps_take_the_prefill_kernel(max_seqlen, D, folds):
+    """Eight new tokens for eight query tokens of 16 heads per KV head (128 rows): the append folds
+    into the decode until the call has enough work for the prefill kernel (12,288 blocks of 32 rows
+    x 64 tokens, 10,240 at head_dim 256; here 192 per 64 tokens of max_seqlen)."""
+    d = base_desc(batch=12, num_heads=64, num_heads_k=4, head_dim=D, page_size=16, block_table_stride=514,
+                  max_seqlen=max_seqlen, num_pages=8192, seqlen_q=8, causal=True)
+    assert pagedkv.append_folds(d, 0, 8) == folds
+    assert pagedkv.append_folds(d, 1, 8) is False  # a forced single pass never folds

@@ -18,9 +18,9 @@ import pytest
 
 import pkv_oracle as po
 from conftest import gpu_available, make_case, rand_bits
-from test_gpu_fp8 import assert_close, f32, fp8_cache, i32, to_dev8
+from test_gpu_fp8 import assert_close, f32, fp8_cache, from_dev8, i32, to_dev8
 from test_gpu_lse import assert_lse, lse_buffer
-from test_gpu_parity import announce, to_dev, torch_mod
+from test_gpu_parity import announce, from_dev, to_dev, torch_mod
 
 pytestmark = [pytest.mark.gpu, pytest.mark.skipif(not gpu_available(), reason="needs a GPU")]
 
@@ -177,3 +177,39 @@ def test_prefill_under_graph_replays():
         torch.cuda.synchronize()
         assert torch.equal(got, want)
         assert torch.equal(call(), want)
+
+
+@pytest.mark.parametrize("D,fp8", [(128, False), (64, True)])
+def test_long_verify_step_appends_then_attends(D, fp8):
+    """A verify step past the fold's work: the new tokens are in the caches bit for bit, the output is
+    the oracle's over the longer rows."""
+    import pagedkv
+
+    torch = torch_mod()
+    announce("prefill-verify", D, fp8)
+    rng = np.random.default_rng(9400 + D)
+    B, H, Hk, P, M, dtype = 3, 32, 2, 16, 8, 1
+    stride = -(-13000 * 64 // (B * Hk * 4)) // P + 1
+    total = np.array([900, 72, 8], np.int32)
+    _, kc, vc, bt, _ = make_case(rng, B=B, H=H, Hk=Hk, D=D, P=P, seqlens=total, dtype=dtype, stride=stride)
+    q = rand_bits(rng, (B, M, H, D), dtype)
+    kn, vn = (rand_bits(rng, (B, M, Hk, D), dtype) for _ in range(2))
+    old = total - M
+    ks = vs = None
+    if fp8:
+        ks, vs = (rng.uniform(0.2, 2.0, Hk).astype(np.float32) for _ in range(2))
+        kc, vc = fp8_cache(rng, kc.shape, ks), fp8_cache(rng, vc.shape, vs)
+        k2, v2 = po.append_kv(kc, vc, bt, old, po.quantize_e4m3(kn, dtype, ks),
+                              po.quantize_e4m3(vn, dtype, vs))
+        want = po.attn8_f64(q, k2, v2, bt, total, 0.1, dtype, k_scale=ks, v_scale=vs, causal=True)
+        kd, vd = to_dev8(kc), to_dev8(vc)
+    else:
+        k2, v2 = po.append_kv(kc, vc, bt, old, kn, vn)
+        want = po.attn_f64(q, k2, v2, bt, total, 0.1, dtype, causal=True)
+        kd, vd = to_dev(kc, dtype), to_dev(vc, dtype)
+    out = pagedkv.decode(to_dev(q, dtype), kd, vd, i32(bt), i32(old), 0.1, 0, k_new=to_dev(kn, dtype),
+                         v_new=to_dev(vn, dtype), causal=True, k_scale=f32(ks), v_scale=f32(vs))
+    torch.cuda.synchronize()
+    assert_close(out, want, dtype)
+    for got, exact in ((kd, k2), (vd, v2)):
+        np.testing.assert_array_equal(from_dev8(got) if fp8 else from_dev(got), exact)
