@@ -429,19 +429,13 @@ __global__ __launch_bounds__(kThreads, D == 256 ? 1 : 2) void prefill_kernel(Par
             if (p.win_right >= 0) {
                 hi = static_cast<int>(min(static_cast<int64_t>(pos) + p.win_right + 1, static_cast<int64_t>(seqlen)));
             }
-            int any_lo = live ? lo : INT32_MAX;
-            int any_hi = live ? hi : 0;
             int all_lo = live ? lo : 0;
             int all_hi = live ? hi : INT32_MAX;
 #pragma unroll
             for (int d = 1; d < 32; d <<= 1) {
-                any_lo = min(any_lo, __shfl_xor(any_lo, d, 64));
-                any_hi = max(any_hi, __shfl_xor(any_hi, d, 64));
                 all_lo = max(all_lo, __shfl_xor(all_lo, d, 64));
                 all_hi = min(all_hi, __shfl_xor(all_hi, d, 64));
             }
-            any_lo = uniform(any_lo);
-            any_hi = uniform(any_hi);
             all_lo = uniform(all_lo);
             all_hi = uniform(all_hi);
             if (!live) {
