@@ -885,22 +885,23 @@ __global__ __launch_bounds__(16 * R) void prefill_combine_kernel(PartitionParams
         acc[e] = 0.f;
     }
     float sum = 0.f;
-    if (mx > kNegInf) {
+    // A part without weight is added too: its row is zeros, or NaN for a query row
+    // that holds a NaN (no part of that row has a weight).
 #pragma unroll 4
-        for (int k = 0; k < cut.parts; ++k) {
-            const int64_t at = slot_row(k);
-            const float wt = fast_exp2(p.part_lse[at] - mx);
-            sum += wt;
-            const float* const src = p.part_o + at * D + 4 * c;
-            float v[E];
+    for (int k = 0; k < cut.parts; ++k) {
+        const int64_t at = slot_row(k);
+        const float lse = p.part_lse[at];
+        const float wt = lse == kNegInf ? 0.f : fast_exp2(lse - mx);
+        sum += wt;
+        const float* const src = p.part_o + at * D + 4 * c;
+        float v[E];
 #pragma unroll
-            for (int e = 0; e < E; e += 4) {
-                *reinterpret_cast<float4*>(v + e) = *reinterpret_cast<const float4*>(src + 16 * e);
-            }
+        for (int e = 0; e < E; e += 4) {
+            *reinterpret_cast<float4*>(v + e) = *reinterpret_cast<const float4*>(src + 16 * e);
+        }
 #pragma unroll
-            for (int e = 0; e < E; ++e) {
-                acc[e] = fmaf(wt, v[e], acc[e]);
-            }
+        for (int e = 0; e < E; ++e) {
+            acc[e] = fmaf(wt, v[e], acc[e]);
         }
     }
     const float inv = sum > 0.f ? 1.f / sum : 0.f;

@@ -18,9 +18,9 @@ import pytest
 
 import pkv_oracle as po
 from conftest import gpu_available, make_case, rand_bits
-from test_gpu_fp8 import assert_close, f32, fp8_cache, from_dev8, i32, to_dev8
+from test_gpu_fp8 import REL, assert_close, f32, fp8_cache, from_dev8, i32, to_dev8
 from test_gpu_lse import assert_lse, lse_buffer
-from test_gpu_parity import announce, from_dev, to_dev, torch_mod
+from test_gpu_parity import TOL, announce, from_dev, to_dev, torch_mod
 
 pytestmark = [pytest.mark.gpu, pytest.mark.skipif(not gpu_available(), reason="needs a GPU")]
 
@@ -213,3 +213,40 @@ def test_long_verify_step_appends_then_attends(D, fp8):
     assert_close(out, want, dtype)
     for got, exact in ((kd, k2), (vd, v2)):
         np.testing.assert_array_equal(from_dev8(got) if fp8 else from_dev(got), exact)
+
+
+@pytest.mark.parametrize("D,M,lens,dtype", [
+    (128, 40, [2100, 1700], 1),          # few streams: cut into many parts
+    (64, 40, [2100, 1700], 0),
+    (256, 40, [2100, 1700], 1),
+    (128, 70, [1 + 7 * (i % 9) for i in range(64)], 0),  # rows of one tile: whole streams
+])
+def test_nan_query_rows_stay_nan(D, M, lens, dtype):
+    """A query row that holds a NaN gives NaN, whether its stream is cut or not, and no other row
+    does."""
+    import pagedkv
+
+    torch = torch_mod()
+    announce("prefill-nan", D, M, len(lens), dtype)
+    rng = np.random.default_rng(9500 + D + M)
+    B, H, Hk, P = len(lens), 16, 4, 16
+    stride = -(-13000 * 64 // (B * Hk * -(-(M * H // Hk) // 32))) // P + 1
+    _, kc, vc, bt, sl = make_case(rng, B=B, H=H, Hk=Hk, D=D, P=P, seqlens=lens, dtype=dtype, stride=stride)
+    q = rand_bits(rng, (B, M, H, D), dtype)
+    nan = rng.random((B, M, H)) < 0.02
+    nan[0, 0, 0] = nan[-1, -1, -1] = True
+    want, want_lse = po.attn_f64(q, kc, vc, bt, sl, 0.1, dtype, lse=True)
+    q[nan, 5] = 0x7FC0 if dtype == 1 else 0x7E00
+    waves, need = desc_plan(q, kc, bt, dtype=dtype)
+    assert need == prefill_workspace(waves, D)
+    lse = lse_buffer(B, H, M)
+    out = pagedkv.decode(to_dev(q, dtype), to_dev(kc, dtype), to_dev(vc, dtype), i32(bt), i32(sl), 0.1, 0,
+                         softmax_lse=lse)
+    torch.cuda.synchronize()
+    got = po.bits_to_f32(from_dev(out), dtype)
+    np.testing.assert_array_equal(np.isnan(got), np.broadcast_to(nan[..., None], got.shape))
+    excess = np.abs(got - want) - (TOL[dtype] + REL[dtype] * np.abs(want))
+    assert np.max(excess[~nan]) < 0
+    lse_nan = nan.transpose(0, 2, 1)
+    want_lse[lse_nan] = np.inf  # as the decode kernels write it
+    assert_lse(lse, want_lse)
