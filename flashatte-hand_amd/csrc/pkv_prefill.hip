@@ -100,24 +100,28 @@ __device__ __forceinline__ uint32_t remainder2(uint32_t heads, float p0, float p
     }
 }
 
-// Tiles of a stream: the 64-token tiles some row of block `hg` can see in a
-// row of `seqlen` tokens.  Window bounds are taken in 64 bits (a window near
-// INT32_MAX must not wrap).
-__device__ __forceinline__ TileSpan prefill_span(const PartitionParams& p, int32_t seqlen, int32_t hg) {
-    const int32_t r0 = hg * kRows;
-    const int32_t r1 = min(p.rows, r0 + kRows) - 1;
-    int64_t lo = 0;
-    int64_t hi = seqlen;
-    if (p.win_left >= 0) {
-        lo = static_cast<int64_t>(seqlen) - p.q_len + r0 / p.group - p.win_left;
-        lo = min(max(lo, int64_t{0}), static_cast<int64_t>(seqlen));
+// The first key that some row of block `hg` can see in a row of `seqlen` tokens.
+// Window bounds are taken in 64 bits (a window near INT32_MAX must not wrap).
+__device__ __forceinline__ int32_t first_visible(const PartitionParams& p, int32_t seqlen, int32_t hg) {
+    if (p.win_left < 0) {
+        return 0;
     }
+    const int64_t lo = static_cast<int64_t>(seqlen) - p.q_len + hg * kRows / p.group - p.win_left;
+    return static_cast<int32_t>(min(max(lo, int64_t{0}), static_cast<int64_t>(seqlen)));
+}
+
+// Tiles of a stream: the 64-token tiles some row of block `hg` can see in a
+// row of `seqlen` tokens.
+__device__ __forceinline__ TileSpan prefill_span(const PartitionParams& p, int32_t seqlen, int32_t hg) {
+    const int32_t r1 = min(p.rows, (hg + 1) * kRows) - 1;
+    const int32_t lo = first_visible(p, seqlen, hg);
+    int64_t hi = seqlen;
     if (p.win_right >= 0) {
         hi = static_cast<int64_t>(seqlen) - p.q_len + r1 / p.group + p.win_right + 1;
         hi = min(max(hi, int64_t{0}), static_cast<int64_t>(seqlen));
     }
     TileSpan t;
-    t.first = static_cast<int32_t>(lo / kPrefillTok);
+    t.first = lo / kPrefillTok;
     t.n = hi > lo ? static_cast<int32_t>((hi + kPrefillTok - 1) / kPrefillTok) - t.first : 0;
     return t;
 }
@@ -418,10 +422,12 @@ __global__ __launch_bounds__(kThreads, D == 256 ? 1 : 2) void prefill_kernel(Par
                 const uint4 v = *reinterpret_cast<const uint4*>(p.q + out_row * D + 16 * kk + 8 * h);
                 q[kk] = make_uint4(v.x ^ flip, v.y ^ flip, v.z ^ flip, v.w ^ flip);
             }
-            // Visible keys [lo, hi) of the lane's row, the wave's bounds, ALiBi.
+            // Visible keys [lo, hi) of the lane's row, the block's first, the wave's
+            // bounds, ALiBi.
             const int pad = p.kv_start != nullptr ? min(max(p.kv_start[b], 0), seqlen) : 0;
+            const int first_key = uniform(max(pad, first_visible(p, seqlen, hg)));
             const int pos = seqlen - p.q_len + qi;
-            int lo = pad;
+            int lo = first_key;
             int hi = seqlen;
             if (p.win_left >= 0) {
                 lo = max(lo, static_cast<int>(max(static_cast<int64_t>(pos) - p.win_left, int64_t{0})));
@@ -461,9 +467,10 @@ __global__ __launch_bounds__(kThreads, D == 256 ? 1 : 2) void prefill_kernel(Par
             float l = 0.f;
 
             // Ends the loads of K passes [kf, kt) and V passes [vf, NP): FP8 rows are converted and stored, and V rows
-            // that no query sees (past the row's end, or padding of
-            // cache_leftpad) cleared: their probability is 0, but they may hold
-            // anything, and 0 times a NaN is a NaN.
+            // that no query of the block sees (past the row's end, padding of
+            // cache_leftpad, or behind the window: the first tile may hold whole
+            // pages that the caller has let go) cleared: their probability is 0,
+            // but they may hold anything, and 0 times a NaN is a NaN.
             const auto finish_rows = [&](int tv, int at, int kf, int kt, int vf) {
                 if constexpr (FP8) {
 #pragma unroll
@@ -475,12 +482,12 @@ __global__ __launch_bounds__(kThreads, D == 256 ? 1 : 2) void prefill_kernel(Par
                         }
                     }
                 }
-                if (tv - 32 < pad || tv + 32 > seqlen) {
+                if (tv - 32 < first_key || tv + 32 > seqlen) {
                     dma_wait();
 #pragma unroll
                     for (int pass = 0; pass < C::NP; ++pass) {
                         const int t = tv - 32 + rr + C::RP * pass;
-                        if (pass >= vf && (t < pad || t >= seqlen)) {
+                        if (pass >= vf && (t < first_key || t >= seqlen)) {
                             *reinterpret_cast<uint4*>(smem + at + 2 * C::kBuf + (rr + C::RP * pass) * D + 8 * cc) =
                                 make_uint4(0u, 0u, 0u, 0u);
                         }

@@ -41,6 +41,11 @@ CASES = [
     (8, 2, 256, 16, [700, 33, 1], 40, dict(causal=True, dtype=0)),
     (4, 2, 256, 32, [400, 320], 100, dict(causal=True, window=(390, 0), softcap=30.0)),
     (8, 2, 256, 64, [300, 65], 40, dict(causal=True, fp8=True)),
+    # Windows whose first tile holds whole pages behind them.
+    (8, 2, 128, 16, [900, 470, 100], 64, dict(causal=True, window=(200, 0), dtype=0)),
+    (8, 2, 128, 16, [900, 490], 64, dict(causal=True, window=(200, 0), fp8=True)),
+    (8, 2, 64, 32, [870, 490], 64, dict(causal=True, window=(200, 0))),
+    (8, 2, 256, 32, [870, 480], 64, dict(causal=False, window=(200, 30), fp8=True, dtype=0)),
 ]
 
 
@@ -55,21 +60,32 @@ def desc_plan(q, kc, bt, **kw):
 
 
 def prefill_workspace(waves, D):
-    assert waves > 0
+    assert waves >= 4  # four a workgroup
     rows = waves // 4 * 2 * 128
     up = lambda x: (x + 255) // 256 * 256  # noqa: E731
     return up(rows * D * 4) + up(rows * 4 + waves // 4 * 16)
 
 
-def hide(kc, vc, bt, lens, leftpad, nan):
-    """Fill every slot that no query sees with `nan`."""
+def hide(kc, vc, bt, lens, first, nan):
+    """Copies with every slot that no query sees (positions below first[b], or past the row) filled with
+    `nan`, and the pages that hold none let go, as an engine does behind a window: their table entries
+    become -1, which the kernels read as page 0, itself made all `nan`."""
+    kc, vc, bt = kc.copy(), vc.copy(), bt.copy()
     P = kc.shape[1]
+    used = {int(bt[b, j]) for b, n in enumerate(lens) for j in range(first[b] // P, -(-max(n, 0) // P))}
+    spare = next(i for i in range(kc.shape[0]) if i not in used)
+    for c in (kc, vc):
+        c[[0, spare]] = c[[spare, 0]]
+    bt[bt == 0] = spare
     seen = np.zeros(kc.shape[:2], bool)
     for b, n in enumerate(lens):
-        t = np.arange(0 if leftpad is None else leftpad[b], max(n, 0))
+        bt[b, :first[b] // P] = -1
+        t = np.arange(first[b], max(n, 0))
         seen[bt[b, t // P], t % P] = True
+    assert not seen[0].any()
     kc[~seen] = nan
     vc[~seen] = nan
+    return kc, vc, bt
 
 
 @pytest.mark.parametrize("case", range(len(CASES)))
@@ -93,6 +109,9 @@ def test_prefill_matches_oracle(case):
     scale = opt.get("scale", 1.0 / math.sqrt(D))
     slopes = rng.uniform(0.01, 0.3, size=(B, H)).astype(np.float32) if opt.get("alibi") else None
     cap = opt.get("softcap", 0.0)
+    first = [0 if leftpad is None else leftpad[b] for b in range(B)]  # the first key some query of the row sees
+    if window[0] >= 0:
+        first = [max(f, n - M - window[0]) for f, n in zip(first, lens)]
     ks = vs = None
     kw = dict(causal=opt["causal"], window=window, alibi=slopes, lse=True, leftpad=None if leftpad is None else
               np.asarray(leftpad, np.int32), softcap=cap)
@@ -100,27 +119,30 @@ def test_prefill_matches_oracle(case):
         ks, vs = (rng.uniform(0.2, 2.0, Hk).astype(np.float32) for _ in range(2))
         kc, vc = fp8_cache(rng, kc.shape, ks), fp8_cache(rng, vc.shape, vs)
         want, want_lse = po.attn8_f64(q, kc, vc, bt, sl, scale, dtype, k_scale=ks, v_scale=vs, **kw)
-        hide(kc, vc, bt, lens, leftpad, 0x7F)
-        kd, vd = to_dev8(kc), to_dev8(vc)
     else:
         want, want_lse = po.attn_f64(q, kc, vc, bt, sl, scale, dtype, **kw)
-        hide(kc, vc, bt, lens, leftpad, 0x7FC0 if dtype == 1 else 0x7E00)
-        kd, vd = to_dev(kc, dtype), to_dev(vc, dtype)
     waves, need = desc_plan(q, kc, bt, dtype=dtype, causal=opt["causal"], window_size=window,
                             kv_dtype=pagedkv.PKV_KV_DTYPE_FP8_E4M3 if fp8 else 0)
     assert need == prefill_workspace(waves, D)
     lse = lse_buffer(B, H, M)
-    args = (to_dev(q, dtype), kd, vd, i32(bt), i32(sl), scale, 0)
+
+    def args(first):
+        k, v, table = hide(kc, vc, bt, lens, first, 0x7F if fp8 else 0x7FC0 if dtype == 1 else 0x7E00)
+        k, v = (to_dev8(k), to_dev8(v)) if fp8 else (to_dev(k, dtype), to_dev(v, dtype))
+        return to_dev(q, dtype), k, v, i32(table), i32(sl), scale, 0
+
     more = dict(causal=opt["causal"], window_size=window, alibi_slopes=f32(slopes), k_scale=f32(ks), v_scale=f32(vs),
                 softcap=cap, cache_leftpad=None if leftpad is None else i32(np.asarray(leftpad, np.int32)))
-    out = pagedkv.decode(*args, softmax_lse=lse, **more)
+    out = pagedkv.decode(*args(first), softmax_lse=lse, **more)
     torch.cuda.synchronize()
     assert_close(out, want, dtype)
     assert_lse(lse, want_lse)
     # A workspace that only the decode kernels' plan fits (1,024 waves' and the streams' slots of 32
-    # rows at most): that plan, within the same tolerance.
+    # rows at most): that plan, within the same tolerance.  Those kernels read from the 16-token tile of
+    # the first key on, behind a window too.
     if need - 256 >= (1024 + B * Hk * -(-(M * H // Hk) // 32)) * 32 * (D + 1) * 4 + 512:
-        small = pagedkv.decode(*args, workspace=torch.empty(need - 256, dtype=torch.uint8, device="cuda"), **more)
+        first = first if leftpad is not None else [f // 16 * 16 for f in first]
+        small = pagedkv.decode(*args(first), workspace=torch.empty(need - 256, dtype=torch.uint8, device="cuda"), **more)
         torch.cuda.synchronize()
         assert_close(small, want, dtype)
 
