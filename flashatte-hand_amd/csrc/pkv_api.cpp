@@ -330,19 +330,24 @@ int64_t prefill_work(const pkv_decode_desc* d, const Resolved& r) {
     return r.B * r.Hk * ((r.rows + 31) / 32) * prefill_tiles(d, r);
 }
 
-// Workgroups of the prefill kernel for this call; 0 = the decode kernels.  Two
-// per CU, one at head_dim 256 (128 KB of LDS).  Beside the work, the kernel's
-// own limits: pages that hold the token rows one load takes, page offsets of 32
-// bits, a plan that fits the LDS and 32-bit units.
+// Whether the prefill kernel is the faster one for this call (with the workspace its plan asks for).
+bool prefill_wins(const pkv_decode_desc* d, const Resolved& r) {
+    return r.rows >= kPrefillMinRows && prefill_work(d, r) >= (r.D == 256 ? kPrefillMinWorkD256 : kPrefillMinWork);
+}
+
+// Workgroups of the prefill kernel for this call, faster or not; 0 = past the
+// kernel's limits: pages that hold the token rows one load takes, page offsets
+// of 32 bits, a plan that fits the LDS and 32-bit units.  Two per CU, one at
+// head_dim 256 (128 KB of LDS).  They grow with the batch, the query tokens and
+// max_seqlen only, so a workspace for a call's plan holds any smaller call's.
 int prefill_groups(const pkv_decode_desc* d, const Resolved& r, int num_splits) {
-    if (num_splits != 0 || d->split_tokens != 0 || r.path != PKV_PATH_MFMA || r.rows < kPrefillMinRows || r.P < 8 ||
+    if (num_splits != 0 || d->split_tokens != 0 || r.path != PKV_PATH_MFMA || r.P < 8 ||
         r.P * r.Hk * r.D * (r.kv_fp8 ? 1 : 2) >= (int64_t{1} << 32)) {
         return 0;
     }
     const int64_t blocks = (r.rows + pkv::kPrefillRows - 1) / pkv::kPrefillRows;
     const int64_t tiles = prefill_tiles(d, r);
-    if (prefill_work(d, r) < (r.D == 256 ? kPrefillMinWorkD256 : kPrefillMinWork) ||
-        r.B * blocks > pkv::kPrefillEntries) {
+    if (r.B * blocks > pkv::kPrefillEntries) {
         return 0;
     }
     // Rows may be longer than max_seqlen: the 32-bit limits are for whole block-table rows.
@@ -364,22 +369,18 @@ int prefill_groups(const pkv_decode_desc* d, const Resolved& r, int num_splits) 
 // 109.0 / 117.1, C4 (513) 127.4 / 130.0, C2 (32) 33.2 / 32.1.
 constexpr int64_t kPairMinShare = 64;
 
-// The plan of a call: the prefill kernel where it applies and its partials fit
-// the `workspace` bytes at hand (a caller whose workspace fits only the decode
-// kernels' plan keeps that one); else resolve_splits, with KV heads paired (r
-// updated) when pairs_ok and the paired plan is the tile schedule with long
-// shares; the single pass, split schedules and the folded append stream one KV
-// head per wave.
-SplitPlan plan_call(const pkv_decode_desc* d, Resolved& r, int num_splits, bool fold,
-                    size_t workspace = SIZE_MAX) {
-    if (!fold) {
-        const int groups = prefill_groups(d, r, num_splits);
-        const SplitPlan plan{PKV_SCHED_TILES, groups * pkv::kTileWaves, 0, groups};
-        if (groups > 0 && workspace_bytes(r, plan) <= workspace) {
-            r.head_groups = static_cast<int>((r.rows + pkv::kPrefillRows - 1) / pkv::kPrefillRows);
-            return plan;
-        }
-    }
+// The prefill kernel's plan, with no workgroups where it cannot take the call
+// or its partials do not fit `workspace` bytes.
+SplitPlan prefill_plan(const pkv_decode_desc* d, const Resolved& r, int num_splits, size_t workspace) {
+    const int groups = prefill_groups(d, r, num_splits);
+    const SplitPlan plan{PKV_SCHED_TILES, groups * pkv::kTileWaves, 0, groups};
+    return groups > 0 && workspace_bytes(r, plan) <= workspace ? plan : SplitPlan{0, 0, 0, 0};
+}
+
+// The decode kernels' plan: resolve_splits, with KV heads paired (r updated)
+// when pairs_ok and the paired plan is the tile schedule with long shares; the
+// single pass, split schedules and the folded append stream one KV head per wave.
+SplitPlan decode_plan(const pkv_decode_desc* d, Resolved& r, int num_splits, bool fold) {
     if (!fold && pairs_ok(r)) {
         const Resolved rp = paired(r);
         const SplitPlan pp = resolve_splits(d, rp, num_splits);
@@ -392,6 +393,26 @@ SplitPlan plan_call(const pkv_decode_desc* d, Resolved& r, int num_splits, bool 
         }
     }
     return resolve_splits(d, r, num_splits);
+}
+
+// The plan of a call with `workspace` bytes at hand (SIZE_MAX: as many as the
+// plan asks for): the prefill kernel where it wins, if its partials fit; else
+// the decode kernels, unless only the prefill kernel's partials fit.  The
+// latter keeps a workspace that was sized for a large prefill enough for every
+// smaller call with the same heads and pages, whose decode plan may need more (32 rows of
+// 40 query tokens, 32/8 heads of 256 dims: 67 MB from 511 tokens on, below
+// them the decode kernels' 76 MB).
+SplitPlan plan_call(const pkv_decode_desc* d, Resolved& r, int num_splits, bool fold,
+                    size_t workspace = SIZE_MAX) {
+    const SplitPlan prefill = fold ? SplitPlan{0, 0, 0, 0} : prefill_plan(d, r, num_splits, workspace);
+    Resolved rd = r;
+    const SplitPlan decode = decode_plan(d, rd, num_splits, fold);
+    if (prefill.prefill > 0 && (prefill_wins(d, r) || workspace_bytes(rd, decode) > workspace)) {
+        r.head_groups = static_cast<int>((r.rows + pkv::kPrefillRows - 1) / pkv::kPrefillRows);
+        return prefill;
+    }
+    r = rd;
+    return decode;
 }
 
 SplitPlan resolve_splits(const pkv_decode_desc* d, const Resolved& r, int num_splits) {
@@ -591,12 +612,12 @@ int decode_impl(const void* q, const void* k_cache, const void* v_cache, const i
     if (num_splits < 0 || !std::isfinite(softmax_scale)) {
         return PKV_EINVAL;
     }
-    const SplitPlan plan =
-        plan_call(desc, r, num_splits, fold != nullptr, desc->workspace != nullptr ? desc->workspace_bytes : 0);
+    const bool usable = desc->workspace != nullptr && aligned16(desc->workspace);
+    const SplitPlan plan = plan_call(desc, r, num_splits, fold != nullptr, usable ? desc->workspace_bytes : 0);
     const bool tiles = plan.schedule == PKV_SCHED_TILES;
     const int splits = tiles ? 0 : plan.splits;
     const size_t need = workspace_bytes(r, plan);
-    if (need > 0 && (desc->workspace == nullptr || desc->workspace_bytes < need || !aligned16(desc->workspace))) {
+    if (need > 0 && (!usable || desc->workspace_bytes < need)) {
         return PKV_ENOWORKSPACE;
     }
     if (fold != nullptr && !fold_plan_ok(r, desc, plan)) {
@@ -784,12 +805,21 @@ pkv::LaunchEvents append_events(const pkv_decode_desc* d) {
     return {ev[0], ev[1]};
 }
 
-// Workspace of pkv_decode_append: the per-row lengths after the append, then
-// the attention's own workspace for the longer rows.
 // Workspace of pkv_decode_append with rotary tables: the rotated q ([B, M, H, D], 16-bit).
 size_t rotary_q_bytes(const Resolved& r) {
     return r.rotary ? align_up(static_cast<size_t>(r.B * r.M * r.H * r.D) * sizeof(uint16_t)) : 0;
 }
+
+// Workspace bytes that the plan queries go by: the descriptor's, or as many as
+// the plan asks for when it has none yet.
+size_t queried_workspace(const pkv_decode_desc* d, size_t head_bytes = 0) {
+    return d->workspace == nullptr ? SIZE_MAX : d->workspace_bytes - std::min(d->workspace_bytes, head_bytes);
+}
+
+// Bytes ahead of the attention's partials in pkv_decode_append's workspace: the
+// per-row lengths, then (rotary) the rotated q.
+size_t append_lens_bytes(const Resolved& r) { return align_up(static_cast<size_t>(r.B) * sizeof(int32_t)); }
+size_t append_head_bytes(const Resolved& r) { return append_lens_bytes(r) + rotary_q_bytes(r); }
 
 pkv_decode_desc appended_desc(const pkv_decode_desc* d, int64_t seqlen_new) {
     pkv_decode_desc a = *d;
@@ -805,13 +835,16 @@ pkv_decode_desc appended_desc(const pkv_decode_desc* d, int64_t seqlen_new) {
 // descriptor `a` without its causal mask (every query sits past them), the
 // combine adds the new tokens each query sees and stores them, and no append
 // kernel runs.  Other calls append first and then attend the longer rows, and so
-// do steps of more than 64 query rows per KV head with the prefill kernel's work.
-bool fold_fits(const pkv_decode_desc* a, int num_splits, int64_t seqlen_new, pkv_decode_desc* part, bool* causal) {
+// do steps of more than 64 query rows per KV head with the prefill kernel's
+// work whose partials fit the `workspace` bytes at hand, or fit them alone (as in plan_call).
+bool fold_fits(const pkv_decode_desc* a, int num_splits, int64_t seqlen_new, size_t workspace, pkv_decode_desc* part,
+               bool* causal) {
     Resolved r;
     if (resolve(a, r) != PKV_OK || seqlen_new != r.M || r.rotary) {
         return false;
     }
-    if (prefill_groups(a, r, num_splits) > 0 && (r.D == 256 || prefill_work(a, r) >= kPrefillMinFoldWork)) {
+    const bool prefill = prefill_plan(a, r, num_splits, workspace).prefill > 0;
+    if (prefill && prefill_wins(a, r) && (r.D == 256 || prefill_work(a, r) >= kPrefillMinFoldWork)) {
         return false;
     }
     *part = *a;
@@ -821,7 +854,8 @@ bool fold_fits(const pkv_decode_desc* a, int num_splits, int64_t seqlen_new, pkv
     if (resolve(part, rp) != PKV_OK) {
         return false;
     }
-    return fold_plan_ok(rp, part, resolve_splits(part, rp, num_splits));
+    const SplitPlan plan = decode_plan(part, rp, num_splits, true);
+    return fold_plan_ok(rp, part, plan) && !(prefill && workspace_bytes(rp, plan) > workspace);
 }
 
 } // namespace
@@ -844,7 +878,7 @@ int pkv_decode_num_splits(const pkv_decode_desc* desc, int num_splits) {
     if (resolve(desc, r) != PKV_OK) {
         return 0;
     }
-    return plan_call(desc, r, num_splits, false).splits;
+    return plan_call(desc, r, num_splits, false, queried_workspace(desc)).splits;
 }
 
 int pkv_decode_split_tokens(const pkv_decode_desc* desc, int num_splits) {
@@ -852,7 +886,7 @@ int pkv_decode_split_tokens(const pkv_decode_desc* desc, int num_splits) {
     if (resolve(desc, r) != PKV_OK) {
         return 0;
     }
-    return plan_call(desc, r, num_splits, false).split_tokens;
+    return plan_call(desc, r, num_splits, false, queried_workspace(desc)).split_tokens;
 }
 
 int pkv_decode_schedule(const pkv_decode_desc* desc, int num_splits) {
@@ -860,7 +894,7 @@ int pkv_decode_schedule(const pkv_decode_desc* desc, int num_splits) {
     if (resolve(desc, r) != PKV_OK) {
         return 0;
     }
-    return plan_call(desc, r, num_splits, false).schedule;
+    return plan_call(desc, r, num_splits, false, queried_workspace(desc)).schedule;
 }
 
 int pkv_decode_path(const pkv_decode_desc* desc) {
@@ -901,8 +935,7 @@ int pkv_decode_noalloc(const void* q, const void* k_cache, const void* v_cache, 
     if (st != PKV_OK) {
         return st;
     }
-    if (num_splits >= 0 &&
-        workspace_bytes(r, plan_call(desc, r, num_splits, false, PKV_SCRATCH_BYTES)) > PKV_SCRATCH_BYTES) {
+    if (num_splits >= 0 && workspace_bytes(r, decode_plan(desc, r, num_splits, false)) > PKV_SCRATCH_BYTES) {
         return PKV_ENOWORKSPACE;
     }
     void* ptr = nullptr;
@@ -988,10 +1021,13 @@ size_t pkv_decode_append_workspace_size(const pkv_decode_desc* desc, int num_spl
     size_t need = pkv_decode_workspace_size(&a, num_splits);
     pkv_decode_desc part;
     bool causal = false;
-    if (fold_fits(&a, num_splits, seqlen_new, &part, &causal)) {
-        need = std::max(need, pkv_decode_workspace_size(&part, num_splits)); // the folded plan's partials
+    if (fold_fits(&a, num_splits, seqlen_new, SIZE_MAX, &part, &causal)) {
+        Resolved rp;
+        (void)resolve(&part, rp); // fold_fits did
+        const SplitPlan plan = decode_plan(&part, rp, num_splits, true);
+        need = std::max(need, workspace_bytes(rp, plan)); // the folded plan's partials
     }
-    return align_up(static_cast<size_t>(r.B) * sizeof(int32_t)) + rotary_q_bytes(r) + need;
+    return append_head_bytes(r) + need;
 }
 
 int pkv_decode_append_folds(const pkv_decode_desc* desc, int num_splits, int64_t seqlen_new) {
@@ -1002,7 +1038,8 @@ int pkv_decode_append_folds(const pkv_decode_desc* desc, int num_splits, int64_t
     const pkv_decode_desc a = appended_desc(desc, seqlen_new);
     pkv_decode_desc part;
     bool causal = false;
-    return fold_fits(&a, num_splits, seqlen_new, &part, &causal) ? 1 : 0;
+    const size_t workspace = queried_workspace(desc, append_head_bytes(r));
+    return fold_fits(&a, num_splits, seqlen_new, workspace, &part, &causal) ? 1 : 0;
 }
 
 int pkv_decode_append(const void* q, const void* k_new, const void* v_new, void* k_cache, void* v_cache,
@@ -1024,10 +1061,7 @@ int pkv_decode_append(const void* q, const void* k_new, const void* v_new, void*
     if (!append_fits(r, seqlen_new)) {
         return PKV_EUNSUPPORTED;
     }
-    // The per-row lengths lead the workspace, then (rotary) the rotated q;
-    // the attention's partials follow.
-    const size_t lens_bytes = align_up(static_cast<size_t>(r.B) * sizeof(int32_t));
-    const size_t head_bytes = lens_bytes + rotary_q_bytes(r);
+    const size_t head_bytes = append_head_bytes(r);
     if (desc->workspace == nullptr || desc->workspace_bytes < head_bytes || !aligned16(desc->workspace)) {
         return PKV_ENOWORKSPACE;
     }
@@ -1040,7 +1074,7 @@ int pkv_decode_append(const void* q, const void* k_new, const void* v_new, void*
     // (two launches instead of three; the lengths region stays unused).
     pkv_decode_desc part;
     bool causal = false;
-    if (fold_fits(&a, num_splits, seqlen_new, &part, &causal)) {
+    if (fold_fits(&a, num_splits, seqlen_new, a.workspace_bytes, &part, &causal)) {
         const AppendFold fold{k_new, v_new, k_cache, v_cache, causal};
         return decode_impl(q, k_cache, v_cache, block_table, cache_seqlens, softmax_scale, num_splits, out, &part,
                            stream, true, &fold);
@@ -1072,7 +1106,7 @@ int pkv_decode_append(const void* q, const void* k_new, const void* v_new, void*
     rp.cos = static_cast<const uint16_t*>(desc->rotary_cos);
     rp.sin = static_cast<const uint16_t*>(desc->rotary_sin);
     rp.q = static_cast<const uint16_t*>(q);
-    rp.q_out = reinterpret_cast<uint16_t*>(static_cast<char*>(desc->workspace) + lens_bytes);
+    rp.q_out = reinterpret_cast<uint16_t*>(static_cast<char*>(desc->workspace) + append_lens_bytes(r));
     rp.rotary_seqlen = desc->rotary_seqlen;
     rp.rotary_dim = desc->rotary_dim;
     rp.interleaved = desc->rotary_interleaved;

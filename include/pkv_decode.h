@@ -155,7 +155,8 @@ typedef struct pkv_decode_desc {
  *       bytes however ragged the rows are (calls with more than 64 query rows
  *       per KV head and enough work: 64-token tiles dealt to workgroups that
  *       share each tile; a workspace that only the waves' partials fit keeps
- *       the waves), and a combine merges the rows that
+ *       the waves, and one that only the workgroups' partials fit takes the
+ *       workgroups), and a combine merges the rows that
  *       more than one wave touched.  Calls too small to fill the chip
  *       (rows of a few tiles, judged from max_seqlen), and calls whose left
  *       window bounds every row, take the single pass instead when its
@@ -177,7 +178,9 @@ int pkv_decode(const void* q, const void* k_cache, const void* v_cache,
                const pkv_decode_desc* desc, void* stream);
 
 /* Bytes of workspace pkv_decode needs for this shape and num_splits (after
- * the same heuristic/clamping pkv_decode applies).  Replaces the reference's
+ * the same heuristic/clamping pkv_decode applies).  Where the kernel for prefill
+ * chunks is chosen, a workspace of that size also serves every call that differs
+ * only by a smaller batch, seqlen_q or max_seqlen.  Replaces the reference's
  * hidden grow-only workspace (best_flashattn_kvcache_decode.cu:17-20, 1078-1133). */
 size_t pkv_decode_workspace_size(const pkv_decode_desc* desc, int num_splits);
 
@@ -213,7 +216,9 @@ int pkv_decode_noalloc(const void* q, const void* k_cache, const void* v_cache,
                        const pkv_decode_desc* desc, void* stream);
 
 /* Split count pkv_decode will use for `num_splits` (0 = heuristic); for
- * PKV_SCHED_TILES, the number of partition waves sharing the tiles.
+ * PKV_SCHED_TILES, the number of partition waves sharing the tiles.  This and the
+ * next two go by desc->workspace_bytes when desc->workspace is set, else by a
+ * workspace of the size pkv_decode_workspace_size returns.
  * Replaces choose_splits (best_flashattn_kvcache_decode.cu:1039-1076, 1299-1312).
  * Returns 0 if desc is invalid. */
 int pkv_decode_num_splits(const pkv_decode_desc* desc, int num_splits);
@@ -300,7 +305,8 @@ size_t pkv_decode_append_workspace_size(const pkv_decode_desc* desc, int num_spl
  * decode step and the speculative verify step, causal or not), 16-bit or
  * FP8 caches, no window, ALiBi, softcap or rotary tables, the tile schedule
  * with its row-per-wave combine, and not so many query rows per KV head (over
- * 64) and tokens that the kernel for prefill chunks is the faster one.  The outputs agree within the decode
+ * 64) and tokens that the kernel for prefill chunks is the faster one (its
+ * workspace at hand: desc->workspace_bytes when desc->workspace is set).  The outputs agree within the decode
  * tolerances (the new tokens' scores are summed in a different order); the
  * caches are written identically.  No
  * counterpart in the reference, whose decode never appends

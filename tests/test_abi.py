@@ -607,3 +607,70 @@ def test_long_verify_steps_take_the_prefill_kernel(max_seqlen, D, folds):
                   max_seqlen=max_seqlen, num_pages=8192, seqlen_q=8, causal=True)
     assert pagedkv.append_folds(d, 0, 8) == folds
     assert pagedkv.append_folds(d, 1, 8) is False  # a forced single pass never folds
+
+
+def plan_bytes(d, bytes_at_hand):
+    """Workspace that pkv_decode's plan needs when it is given `bytes_at_hand`."""
+    D = d.head_dim
+    align = lambda x: (x + 255) // 256 * 256  # noqa: E731
+    asked, need = pagedkv.num_splits_for(d, 0), pagedkv.workspace_size(d, 0)
+    d.workspace, d.workspace_bytes = 4096, bytes_at_hand
+    waves = pagedkv.num_splits_for(d, 0)
+    d.workspace, d.workspace_bytes = None, 0
+    if need <= bytes_at_hand or (waves == asked and D != 256):  # at head_dim 256 both plans may have 1,024 waves
+        return need
+    rows = waves // 4 * 2 * 128  # the other plan: the prefill kernel's
+    return align(rows * D * 4) + align(rows * 4 + waves // 4 * 16)
+
+
+@pytest.mark.parametrize("H,Hk,D,B,M,max_seqlen", [
+    (32, 8, 256, 32, 40, 8192),   # the decode plan of up to 448 tokens needs 76 MB, this call's plan 67 MB
+    (32, 8, 256, 32, 40, 511),
+    (32, 8, 128, 256, 100, 2048),
+    (128, 32, 64, 180, 40, 1024),
+    (8, 8, 128, 100, 512, 4096),
+    (64, 2, 128, 500, 9, 700),
+])
+def test_workspace_of_a_prefill_call_serves_every_smaller_call(H, Hk, D, B, M, max_seqlen):
+    """A caller may size its workspace once, for its largest call: no call that differs by a smaller
+    batch, seqlen_q or max_seqlen is then refused."""
+    kw = dict(num_heads=H, num_heads_k=Hk, head_dim=D, page_size=16, block_table_stride=512, num_pages=4096,
+              causal=True)
+    at_hand = pagedkv.workspace_size(base_desc(batch=B, seqlen_q=M, max_seqlen=max_seqlen, **kw), 0)
+    for b in (B, B - 1, B // 2, B // 7, 1):
+        for m in (M, M // 2, M // 5, 2, 1):
+            for n in (max_seqlen, max_seqlen // 2, 449, 448, 128, 64, 16, 1):
+                if m >= 1 and n <= max_seqlen:
+                    d = base_desc(batch=b, seqlen_q=m, max_seqlen=n, **kw)
+                    assert plan_bytes(d, at_hand) <= at_hand, (b, m, n)
+
+
+def test_plan_queries_go_by_the_workspace_at_hand():
+    """With a workspace that only one of the two plans fits the queries report that plan, as pkv_decode
+    takes it; a workspace size query is always that of the plan taken without such a limit."""
+    d = base_desc(batch=4, num_heads=32, page_size=16, block_table_stride=512, max_seqlen=8192, num_pages=4096,
+                  seqlen_q=64)
+    waves, need = pagedkv.num_splits_for(d, 0), pagedkv.workspace_size(d, 0)
+    assert waves == 2048  # 512 workgroups of the prefill kernel
+    for at_hand, expected in ((need, 2048), (need - 1, 1024)):
+        d.workspace, d.workspace_bytes = 4096, at_hand
+        assert pagedkv.num_splits_for(d, 0) == expected
+        assert pagedkv.schedule_for(d, 0) == pagedkv.PKV_SCHED_TILES
+        assert pagedkv.workspace_size(d, 0) == need
+
+
+def test_folded_append_stays_where_only_its_workspace_is_at_hand():
+    """A verify step with the prefill kernel's work, in a workspace that holds the folded plan's
+    partials but not the prefill kernel's: the append folds, as it does below that work."""
+    align = lambda x: (x + 255) // 256 * 256  # noqa: E731
+    d = base_desc(batch=12, num_heads=64, num_heads_k=4, head_dim=128, page_size=16, block_table_stride=514,
+                  max_seqlen=5000, num_pages=8192, seqlen_q=8, causal=True)
+    assert pagedkv.append_folds(d, 0, 8) is False
+    rows = (1024 + 12 * 4 * 4) * 32  # waves and streams (4 head groups of 32 rows) of the folded plan
+    fold = align(rows * 128 * 4) + align(rows * 4)
+    lens = align(12 * 4)
+    full = _lib.load().pkv_decode_append_workspace_size(ctypes.byref(d), 0, 8)
+    assert fold < full - lens
+    for at_hand, folds in ((lens + fold, True), (full - 1, True), (full, False)):
+        d.workspace, d.workspace_bytes = 4096, at_hand
+        assert pagedkv.append_folds(d, 0, 8) is folds, at_hand

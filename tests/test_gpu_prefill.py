@@ -272,3 +272,73 @@ def test_nan_query_rows_stay_nan(D, M, lens, dtype):
     lse_nan = nan.transpose(0, 2, 1)
     want_lse[lse_nan] = np.inf  # as the decode kernels write it
     assert_lse(lse, want_lse)
+
+
+@pytest.mark.parametrize("H,Hk,D,B,M,bound,longest,dtype,opt", [
+    (32, 8, 256, 32, 40, 511, 128, 1, dict(causal=True)),
+    (128, 32, 64, 180, 5, 1024, 70, 0, dict(causal=True)),                    # 20 query rows per KV head
+    (128, 32, 64, 180, 5, 1024, 70, 1, dict(causal=True, window=(50, 0))),
+    (64, 32, 128, 110, 17, 1024, 40, 1, dict(causal=False, fp8=True)),         # 34 rows
+])
+def test_workspace_sized_for_longer_rows(H, Hk, D, B, M, bound, longest, dtype, opt):
+    """A workspace sized for a large prefill, given to a call of short rows or few query tokens whose
+    decode plan needs more: the call takes the prefill kernel instead of being refused."""
+    import pagedkv
+
+    torch = torch_mod()
+    announce("prefill-small-workspace", H, Hk, D, B, M, bound, longest, dtype, opt)
+    rng = np.random.default_rng(9600 + D + M)
+    P, fp8, causal, window = 16, opt.get("fp8", False), opt["causal"], opt.get("window", (-1, -1))
+    lens = rng.integers(0, longest + 1, size=B).astype(np.int32)
+    lens[:3] = (0, 1, longest)
+    _, kc, vc, bt, sl = make_case(rng, B=B, H=H, Hk=Hk, D=D, P=P, seqlens=lens, dtype=dtype, stride=bound // P)
+    q = rand_bits(rng, (B, M, H, D), dtype)
+    kv_dtype = pagedkv.PKV_KV_DTYPE_FP8_E4M3 if fp8 else 0
+    at_hand = desc_plan(rand_bits(rng, (B, max(M, 40), 1, D), dtype).repeat(H, axis=2), kc, bt, dtype=dtype, causal=True,
+                        max_seqlen=bound, kv_dtype=kv_dtype)[1]
+    waves, need = desc_plan(q, kc, bt, dtype=dtype, causal=causal, window_size=window, max_seqlen=longest,
+                            kv_dtype=kv_dtype)
+    assert need > at_hand
+    ks = vs = None
+    if fp8:
+        ks, vs = (rng.uniform(0.2, 2.0, Hk).astype(np.float32) for _ in range(2))
+        kc, vc = fp8_cache(rng, kc.shape, ks), fp8_cache(rng, vc.shape, vs)
+        want, want_lse = po.attn8_f64(q, kc, vc, bt, sl, 0.1, dtype, k_scale=ks, v_scale=vs, causal=causal,
+                                      window=window, lse=True)
+    else:
+        want, want_lse = po.attn_f64(q, kc, vc, bt, sl, 0.1, dtype, causal=causal, window=window, lse=True)
+    lse = lse_buffer(B, H, M)
+    out = pagedkv.decode(to_dev(q, dtype), to_dev8(kc) if fp8 else to_dev(kc, dtype),
+                         to_dev8(vc) if fp8 else to_dev(vc, dtype), i32(bt), i32(sl), 0.1, 0, causal=causal,
+                         window_size=window, max_seqlen=longest, k_scale=f32(ks), v_scale=f32(vs), softmax_lse=lse,
+                         workspace=torch.empty(at_hand, dtype=torch.uint8, device="cuda"))
+    torch.cuda.synchronize()
+    assert_close(out, want, dtype)
+    assert_lse(lse, want_lse)
+
+
+def test_verify_step_folds_in_a_workspace_for_the_fold():
+    """A verify step with the prefill kernel's work, given a workspace that holds only the folded
+    plan's partials: the oracle's output, the new tokens in the caches bit for bit."""
+    import pagedkv
+
+    torch = torch_mod()
+    announce("prefill-verify-fold-workspace")
+    rng = np.random.default_rng(9700)
+    B, H, Hk, D, P, M, dtype = 3, 32, 2, 128, 16, 8, 1
+    stride = -(-13000 * 64 // (B * Hk * 4)) // P + 1
+    total = np.array([900, 72, 8], np.int32)
+    _, kc, vc, bt, _ = make_case(rng, B=B, H=H, Hk=Hk, D=D, P=P, seqlens=total, dtype=dtype, stride=stride)
+    q = rand_bits(rng, (B, M, H, D), dtype)
+    kn, vn = (rand_bits(rng, (B, M, Hk, D), dtype) for _ in range(2))
+    k2, v2 = po.append_kv(kc, vc, bt, total - M, kn, vn)
+    want = po.attn_f64(q, k2, v2, bt, total, 0.1, dtype, causal=True)
+    rows = (1024 + B * Hk * 4) * 32
+    workspace = torch.empty(256 + rows * D * 4 + rows * 4, dtype=torch.uint8, device="cuda")
+    kd, vd = to_dev(kc, dtype), to_dev(vc, dtype)
+    out = pagedkv.decode(to_dev(q, dtype), kd, vd, i32(bt), i32(total - M), 0.1, 0, k_new=to_dev(kn, dtype),
+                         v_new=to_dev(vn, dtype), causal=True, workspace=workspace)
+    torch.cuda.synchronize()
+    assert_close(out, want, dtype)
+    for got, exact in ((kd, k2), (vd, v2)):
+        np.testing.assert_array_equal(from_dev(got), exact)
