@@ -200,10 +200,14 @@ size_t pkv_decode_workspace_size(const pkv_decode_desc* desc, int num_splits);
  * its first pkv_decode call take 0 and 6 MiB of device memory, the first
  * pkv_decode_noalloc call 34 MiB more; callers that never use this entry point
  * do not pay for the buffer.
- * - A plan that needs more than PKV_SCRATCH_BYTES
- *   (pkv_decode_workspace_size(desc, num_splits) > PKV_SCRATCH_BYTES, e.g.
- *   forced splits over very many rows) returns PKV_ENOWORKSPACE before anything
- *   is enqueued; the heuristic plans of the benchmark configs need at most 21 MB.
+ * - A call whose plan on the decode kernels needs more than PKV_SCRATCH_BYTES
+ *   (e.g. forced splits over very many rows) returns PKV_ENOWORKSPACE before
+ *   anything is enqueued; the heuristic plans of the benchmark configs need at
+ *   most 21 MB.  Where pkv_decode takes the kernel for prefill chunks,
+ *   pkv_decode_workspace_size returns that kernel's need (up to 68 MB) and says
+ *   nothing about this call: it takes that kernel if its partials fit the
+ *   scratch, else the decode kernels.  (The plan queries below report which, with
+ *   desc->workspace set and desc->workspace_bytes = PKV_SCRATCH_BYTES.)
  * - `stream` must belong to the current device (PKV_EINVAL otherwise).
  * - Every call on one GPU shares that GPU's buffer: calls that overlap on one
  *   GPU (on other streams, from other host threads) race; serialise them.

@@ -317,6 +317,27 @@ def test_workspace_sized_for_longer_rows(H, Hk, D, B, M, bound, longest, dtype, 
     assert_lse(lse, want_lse)
 
 
+def test_misaligned_workspace_where_none_is_needed():
+    """Rows bounded by a window: the decode kernels' plan is the single pass, so a workspace that the
+    prefill kernel cannot use does not stop the call."""
+    import pagedkv
+
+    torch = torch_mod()
+    announce("prefill-misaligned-workspace")
+    rng = np.random.default_rng(9650)
+    B, H, Hk, D, P, M, dtype, window = 16, 64, 16, 128, 16, 64, 1, (200, 0)
+    _, kc, vc, bt, sl = make_case(rng, B=B, H=H, Hk=Hk, D=D, P=P, seqlens=[900, 490] * 8, dtype=dtype)
+    q = rand_bits(rng, (B, M, H, D), dtype)
+    waves, need = desc_plan(q, kc, bt, dtype=dtype, causal=True, window_size=window)
+    assert need == prefill_workspace(waves, D)
+    want = po.attn_f64(q, kc, vc, bt, sl, 0.1, dtype, causal=True, window=window)
+    out = pagedkv.decode(to_dev(q, dtype), to_dev(kc, dtype), to_dev(vc, dtype), i32(bt), i32(sl), 0.1, 0,
+                         causal=True, window_size=window,
+                         workspace=torch.empty(need + 16, dtype=torch.uint8, device="cuda")[8:])
+    torch.cuda.synchronize()
+    assert_close(out, want, dtype)
+
+
 def test_verify_step_folds_in_a_workspace_for_the_fold():
     """A verify step with the prefill kernel's work, given a workspace that holds only the folded
     plan's partials: the oracle's output, the new tokens in the caches bit for bit."""

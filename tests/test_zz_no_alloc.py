@@ -3,7 +3,7 @@ caller workspace.  Through the C ABI, against pkv_decode with a caller workspace
 and plan, so the bits must agree), on two calls in a row, the second with a smaller input (fewer,
 shorter rows: the scratch still holds the first call's partials), over the heuristic tile
 schedule, page splits and token windows; and a plan larger than the scratch is refused before
-anything is enqueued.
+anything is enqueued.  Prefill chunks run whether the prefill kernel's partials fit the scratch or not.
 """
 from __future__ import annotations
 
@@ -14,7 +14,7 @@ import numpy as np
 import pytest
 
 import pkv_oracle as po
-from conftest import gpu_available, make_case
+from conftest import gpu_available, make_case, rand_bits
 from test_gpu_parity import TOL, announce, from_dev, to_dev, torch_mod
 
 pytestmark = [pytest.mark.gpu, pytest.mark.skipif(not gpu_available(), reason="needs a GPU")]
@@ -91,6 +91,42 @@ def test_noalloc_matches_pkv_decode_on_two_calls(plan):
         err = float(np.max(np.abs(po.bits_to_f32(got, dtype) - want)))
         print(f"{name}: max_abs_err={err:.3e}", flush=True)
         assert err < TOL[dtype], name
+
+
+@pytest.mark.parametrize("D,dtype,fits", [(128, 1, False), (64, 1, True)])
+def test_noalloc_takes_prefill_chunks(D, dtype, fits):
+    """A call with the prefill kernel's work, whose workspace size is past the scratch at head_dim 128
+    (the decode kernels' plan, which fits, then runs) and within it here at 64: the oracle's output either
+    way, and the plan queries say which plan it is."""
+    import pagedkv
+    from pagedkv import _lib
+
+    torch = torch_mod()
+    announce("noalloc-prefill", D, dtype, fits)
+    rng = np.random.default_rng(3400 + D)
+    H, Hk, P, M = 32, 8, 16, 64
+    lens = [900] if fits else [700, 65, 300, 0]
+    width = 8320 // P if fits else 4096 // P
+    _, k, v, bt, sl = make_case(rng, B=len(lens), H=H, Hk=Hk, D=D, P=P, seqlens=lens, dtype=dtype, stride=width)
+    q = rand_bits(rng, (len(lens), M, H, D), dtype)
+    desc = pagedkv.make_desc(batch=len(lens), num_heads=H, num_heads_k=Hk, head_dim=D, page_size=P,
+                             num_pages=k.shape[0], block_table_stride=width, dtype=dtype, seqlen_q=M, causal=True)
+    need, asked = pagedkv.workspace_size(desc), pagedkv.num_splits_for(desc)
+    assert need == -(-asked // 4 * 256 * D * 4 // 256) * 256 + -(-(asked // 4 * (256 * 4 + 16)) // 256) * 256
+    assert (need <= _lib.PKV_SCRATCH_BYTES) == fits
+    desc.workspace, desc.workspace_bytes = 4096, _lib.PKV_SCRATCH_BYTES  # for the query only
+    waves = pagedkv.num_splits_for(desc)
+    assert waves == asked if fits else waves < asked
+    desc.workspace, desc.workspace_bytes = None, 0
+    dq, dk, dv, dbt, dsl = to_dev(q, dtype), to_dev(k, dtype), to_dev(v, dtype), i32(bt), i32(sl)
+    out = torch.full_like(dq, float("nan"))
+    st = _lib.load().pkv_decode_noalloc(dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dbt.data_ptr(), dsl.data_ptr(),
+                                        0.1, 0, out.data_ptr(), ctypes.byref(desc),
+                                        torch.cuda.current_stream().cuda_stream)
+    assert st == 0, _lib.strerror(st)
+    torch.cuda.synchronize()
+    want = po.attn_f64(q, k, v, bt, sl, 0.1, dtype, causal=True)
+    assert float(np.max(np.abs(po.bits_to_f32(from_dev(out), dtype) - want))) < TOL[dtype]
 
 
 def test_noalloc_refuses_plans_larger_than_the_scratch():
