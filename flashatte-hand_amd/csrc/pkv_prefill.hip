@@ -171,12 +171,16 @@ struct Prefill {
 // (wave-uniform base and lds).  Counted by vmcnt, which the compiler does not
 // know here: dma_wait() before the barrier that publishes the tile.  It writes
 // a buffer that nobody reads before that barrier, so reads may pass it.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm" // m0 is a reserved register: its clobber is declared all the same
 __device__ __forceinline__ void dma16(uint64_t base, uint32_t off, uint32_t lds) {
     // Five wait states: base may come from a lane read just before.
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %2"
                  :
-                 : "s"(lds), "v"(off), "s"(base));
+                 : "s"(lds), "v"(off), "s"(base)
+                 : "m0");
 }
+#pragma clang diagnostic pop
 __device__ __forceinline__ void dma_wait() { asm volatile("s_waitcnt vmcnt(0)" : : : "memory"); }
 
 typedef __attribute__((address_space(3))) uint16_t lds_u16;

@@ -674,3 +674,14 @@ def test_folded_append_stays_where_only_its_workspace_is_at_hand():
     for at_hand, folds in ((lens + fold, True), (full - 1, True), (full, False)):
         d.workspace, d.workspace_bytes = 4096, at_hand
         assert pagedkv.append_folds(d, 0, 8) is folds, at_hand
+
+
+def test_inline_assembly_declares_m0():
+    """Every asm statement of the kernels that writes m0 names it among its clobbers."""
+    seen = 0
+    for src in sorted((HEADER.parent.parent / "flashatte-hand_amd" / "csrc").iterdir()):
+        for stmt in re.findall(r"\basm\b.*?\);", src.read_text(), flags=re.S):
+            if re.search(r"\bs_mov_b32\s+m0\b", stmt):
+                seen += 1
+                assert re.search(r':[^:]*"m0"[^:]*\);$', stmt), (src.name, stmt)
+    assert seen > 0
