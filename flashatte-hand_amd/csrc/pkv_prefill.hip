@@ -247,7 +247,18 @@ __global__ __launch_bounds__(kThreads, D == 256 ? 1 : 2) void prefill_kernel(Par
         __syncthreads();
     }
     const uint32_t total = uniform(static_cast<int32_t>(prefix[entries])) * static_cast<uint32_t>(hk); // < 2^31 (host rule)
-    const int32_t workers = static_cast<int32_t>(min(static_cast<uint32_t>(launched), total));
+    // Workgroups with a share.  The launch is sized from max_seqlen, and rows may
+    // be far shorter; a smaller share then cuts the streams into more parts than
+    // their merge is worth.  With u units per stream a share has at least
+    // sqrt(u) / 4 units, and 3 where that still leaves one workgroup per CU.  Measured
+    // (head_dim 64, 8 query tokens x 16 heads per KV head, table of 131,072 tokens; shares
+    // of one unit or more / this / the decode kernels, us): 8 streams of 64 tiles 32 / 28 /
+    // 22.5, 2 of 256 tiles 46 / 28 / 21, 32 of 16 tiles 30 / 26 / 22.7.
+    const float per_stream = static_cast<float>(total) / static_cast<float>(entries * hk);
+    const float most = fminf(static_cast<float>(launched),
+                             fmaxf(static_cast<float>(kComputeUnits), static_cast<float>(total) * (1.f / 3.f)));
+    const float least = fmaxf(1.f, 0.25f * sqrtf(per_stream)); // units per share
+    const int32_t workers = uniform(max(1, static_cast<int32_t>(fminf(most, static_cast<float>(total) / least))));
     if (w >= workers) {
         if (tid == 0) {
             cuts[w] = CutStream{0, 0, 0, 0};
@@ -865,31 +876,34 @@ __global__ __launch_bounds__(kThreads, D == 256 ? 1 : 2) void prefill_kernel(Par
 
 // Merges the cut streams: workgroup (i, w) takes rows R i .. R (i + 1) - 1 of
 // the stream whose first part workgroup w of the partition left, if any.  16
-// lanes per row; the parts' weights come from their log2-domain LSEs.  Bound:
-// the partials' bytes; and, with R = 8, the dispatch of the workgroups.
-template <bool BF16, int D, int R>
-__global__ __launch_bounds__(16 * R) void prefill_combine_kernel(PartitionParams p) {
+// lanes per row; the parts' weights come from their log2-domain LSEs.  W slices
+// of the workgroup take every W-th part each and are added through the LDS: a
+// long stream cut over the whole chip has hundreds of parts, which one slice
+// walks a round trip at a time (512 parts of 2 streams, head_dim 64: the call
+// 77 us, with four slices 46).  Bound: the partials' bytes; and the dispatch of
+// the workgroups.
+template <bool BF16, int D, int R, int W>
+__global__ __launch_bounds__(16 * R * W) void prefill_combine_kernel(PartitionParams p) {
     constexpr int E = D / 16; // dims per lane, four at a time: 64 e / 4 + 4 c ..
     const int w = static_cast<int>(blockIdx.y);
     const CutStream cut =
         reinterpret_cast<const CutStream*>(p.part_lse + static_cast<int64_t>(p.tile_workers) * 2 * kRows)[w];
-    if (cut.parts == 0) {
+    const int r0 = cut.hg * kRows + static_cast<int>(blockIdx.x) * R;
+    if (cut.parts == 0 || r0 >= p.rows) {
         return;
     }
     const int c = threadIdx.x & 15;
-    const int row = static_cast<int>(blockIdx.x) * R + static_cast<int>(threadIdx.x) / 16;
-    const int r = cut.hg * kRows + row;
-    if (r >= p.rows) {
-        return;
-    }
+    const int slice = static_cast<int>(threadIdx.x) / (16 * R);
+    const int r = min(r0 + static_cast<int>(threadIdx.x) / 16 % R, p.rows - 1); // past the rows: the last one again
+    const int row = r - cut.hg * kRows;
     const auto slot_row = [&](int k) {
         return static_cast<int64_t>(k == 0 ? 2 * w + 1 : 2 * (w + k)) * kRows + row;
     };
     float mx = kNegInf;
-#pragma unroll 4
-    for (int k = 0; k < cut.parts; ++k) {
+    for (int k = c; k < cut.parts; k += 16) {
         mx = fmaxf(mx, p.part_lse[slot_row(k)]);
     }
+    mx = group_max<16>(mx);
     float acc[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) {
@@ -899,7 +913,7 @@ __global__ __launch_bounds__(16 * R) void prefill_combine_kernel(PartitionParams
     // A part without weight is added too: its row is zeros, or NaN for a query row
     // that holds a NaN (no part of that row has a weight).
 #pragma unroll 4
-    for (int k = 0; k < cut.parts; ++k) {
+    for (int k = slice; k < cut.parts; k += W) {
         const int64_t at = slot_row(k);
         const float lse = p.part_lse[at];
         const float wt = lse == kNegInf ? 0.f : fast_exp2(lse - mx);
@@ -913,6 +927,29 @@ __global__ __launch_bounds__(16 * R) void prefill_combine_kernel(PartitionParams
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             acc[e] = fmaf(wt, v[e], acc[e]);
+        }
+    }
+    if constexpr (W > 1) {
+        __shared__ float other[W - 1][E + 1][16 * R];
+        const int at = static_cast<int>(threadIdx.x) % (16 * R);
+        if (slice > 0) {
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                other[slice - 1][e][at] = acc[e];
+            }
+            other[slice - 1][E][at] = sum;
+        }
+        __syncthreads();
+        if (slice > 0) {
+            return;
+        }
+#pragma unroll
+        for (int i = 0; i < W - 1; ++i) {
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                acc[e] += other[i][e][at];
+            }
+            sum += other[i][E][at];
         }
     }
     const float inv = sum > 0.f ? 1.f / sum : 0.f;
@@ -950,10 +987,11 @@ hipError_t launch_d(const PartitionParams& p, hipStream_t stream, const LaunchEv
     // Few streams of many parts each need the workgroups; many cut streams fill
     // the chip as it is, and fewer workgroups are dispatched.
     if (p.batch * p.num_heads_k * p.head_groups > kComputeUnits / 2) {
-        launch_kernel(prefill_combine_kernel<BF16, D, 16>, dim3(kRows / 16, p.tile_workers), dim3(256), 0, stream, comb_ev,
-                      p);
+        launch_kernel(prefill_combine_kernel<BF16, D, 16, 1>, dim3(kRows / 16, p.tile_workers), dim3(256), 0, stream,
+                      comb_ev, p);
     } else {
-        launch_kernel(prefill_combine_kernel<BF16, D, 4>, dim3(kRows / 4, p.tile_workers), dim3(64), 0, stream, comb_ev, p);
+        launch_kernel(prefill_combine_kernel<BF16, D, 4, 4>, dim3(kRows / 4, p.tile_workers), dim3(256), 0, stream, comb_ev,
+                      p);
     }
     return hipGetLastError();
 }

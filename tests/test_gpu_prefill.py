@@ -41,6 +41,10 @@ CASES = [
     (8, 2, 256, 16, [700, 33, 1], 40, dict(causal=True, dtype=0)),
     (4, 2, 256, 32, [400, 320], 100, dict(causal=True, window=(390, 0), softcap=30.0)),
     (8, 2, 256, 64, [300, 65], 40, dict(causal=True, fp8=True)),
+    # Few streams over a table far wider than the rows: 70 to 130 parts each.
+    (16, 1, 64, 256, [20000], 8, dict(causal=True)),
+    (16, 1, 128, 64, [16000, 5000], 8, dict(causal=True, fp8=True, dtype=0)),
+    (16, 1, 256, 16, [9000], 9, dict(causal=True, softcap=20.0, dtype=0)),
     # Windows whose first tile holds whole pages behind them.
     (8, 2, 128, 16, [900, 470, 100], 64, dict(causal=True, window=(200, 0), dtype=0)),
     (8, 2, 128, 16, [900, 490], 64, dict(causal=True, window=(200, 0), fp8=True)),
