@@ -573,7 +573,10 @@ def test_head_groups_share_a_gang_on_the_tile_schedule():
     ({"batch": 1}, True),
     ({"page_size": 4}, False),               # a load's token rows would span pages
     ({"split_tokens": 512}, False),
-    ({"path": pagedkv.PKV_PATH_VALU, "seqlen_q": 1}, False),
+    ({"num_heads": 576, "seqlen_q": 1}, True),  # 72 heads per KV head, one query token
+    ({"num_heads": 576, "seqlen_q": 1, "path": pagedkv.PKV_PATH_VALU}, False),
+    ({"batch": 1024, "max_seqlen": 512}, True),    # 1,024 rows of two row blocks: all the plan's entries
+    ({"batch": 1025, "max_seqlen": 512}, False),
 ])
 def test_prefill_kernel_in_the_plan(change, prefill):
     """Calls with more than 64 query rows per KV head and enough 32-row x 64-token blocks of work

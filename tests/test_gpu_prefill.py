@@ -41,6 +41,19 @@ CASES = [
     (8, 2, 256, 16, [700, 33, 1], 40, dict(causal=True, dtype=0)),
     (4, 2, 256, 32, [400, 320], 100, dict(causal=True, window=(390, 0), softcap=30.0)),
     (8, 2, 256, 64, [300, 65], 40, dict(causal=True, fp8=True)),
+    # Every layout of the capped slots, past the masked blocks of a row's end; with ALiBi every block is
+    # capped ahead of them.
+    (8, 2, 64, 16, [700, 130], 40, dict(causal=True, softcap=8.0)),
+    (8, 2, 64, 16, [700, 130], 40, dict(causal=True, softcap=8.0, dtype=0)),
+    (8, 2, 64, 16, [700, 130], 40, dict(causal=True, softcap=8.0, fp8=True)),
+    (8, 2, 128, 16, [700, 130], 40, dict(causal=True, softcap=8.0, fp8=True, dtype=0)),
+    (8, 2, 256, 16, [700, 130], 40, dict(causal=True, softcap=8.0, fp8=True)),
+    (8, 2, 64, 16, [700, 130], 40, dict(causal=False, softcap=8.0, alibi=True)),
+    (8, 2, 64, 16, [700, 130], 40, dict(causal=True, dtype=0)),
+    # One query token, many heads per KV head: a decode step of the same kernel.
+    (128, 1, 128, 16, [900, 1, 0, 333], 1, dict(causal=False)),
+    (142, 2, 64, 64, [900, 65], 1, dict(causal=True, dtype=0)),
+    (96, 1, 256, 32, [500, 64], 1, dict(causal=False, fp8=True)),
     # Few streams over a table far wider than the rows: 70 to 130 parts each.
     (16, 1, 64, 256, [20000], 8, dict(causal=True)),
     (16, 1, 128, 64, [16000, 5000], 8, dict(causal=True, fp8=True, dtype=0)),
@@ -173,6 +186,26 @@ def test_prefill_many_ragged_rows():
     assert_close(out, want, dtype)
 
 
+def test_prefill_at_its_limit_of_row_blocks():
+    """1,024 rows of two row blocks: as many entries as the plan in the LDS holds."""
+    import pagedkv
+
+    torch = torch_mod()
+    announce("prefill-entries")
+    rng = np.random.default_rng(9250)
+    B, H, Hk, D, P, M, dtype = 1024, 4, 1, 64, 16, 33, 0
+    lens = rng.integers(0, 129, size=B).astype(np.int32)
+    _, kc, vc, bt, sl = make_case(rng, B=B, H=H, Hk=Hk, D=D, P=P, seqlens=lens, dtype=dtype, stride=8)
+    q = rand_bits(rng, (B, M, H, D), dtype)
+    want = po.attn_f64(q, kc, vc, bt, sl, 0.12, dtype, causal=True)
+    waves, need = desc_plan(q, kc, bt, dtype=dtype, causal=True)
+    assert need == prefill_workspace(waves, D)
+    out = pagedkv.decode(to_dev(q, dtype), to_dev(kc, dtype), to_dev(vc, dtype), i32(bt), i32(sl), 0.12, 0,
+                         causal=True)
+    torch.cuda.synchronize()
+    assert_close(out, want, dtype)
+
+
 def test_prefill_under_graph_replays():
     """A captured appending prefill chunk, replayed several times with eager work in between."""
     import pagedkv
@@ -181,15 +214,21 @@ def test_prefill_under_graph_replays():
     announce("prefill-graph")
     rng = np.random.default_rng(9300)
     B, H, Hk, D, P, M, dtype = 2, 32, 8, 128, 16, 96, 1
-    _, kc, vc, bt, sl = make_case(rng, B=B, H=H, Hk=Hk, D=D, P=P, seqlens=[1500, 700], dtype=dtype)
-    q, kd, vd = to_dev(rand_bits(rng, (B, M, H, D), dtype), dtype), to_dev(kc, dtype), to_dev(vc, dtype)
-    kn, vn = (to_dev(rand_bits(rng, (B, M, Hk, D), dtype), dtype) for _ in range(2))
+    _, kc, vc, bt, sl = make_case(rng, B=B, H=H, Hk=Hk, D=D, P=P, seqlens=[1500, 700], dtype=dtype, stride=200)
+    q, kn, vn = rand_bits(rng, (B, M, H, D), dtype), *(rand_bits(rng, (B, M, Hk, D), dtype) for _ in range(2))
+    waves, need = desc_plan(q, kc, bt, dtype=dtype, causal=True)
+    assert need == prefill_workspace(waves, D)
+    k2, v2 = po.append_kv(kc, vc, bt, np.asarray(sl) - M, kn, vn)
+    exact = po.attn_f64(q, k2, v2, bt, sl, 0.09, dtype, causal=True)
+    q, kn, vn, kd, vd = (to_dev(t, dtype) for t in (q, kn, vn, kc, vc))
     table, lens = i32(bt), i32(np.asarray(sl) - M)
 
     def call():
         return pagedkv.decode(q, kd, vd, table, lens, 0.09, 0, k_new=kn, v_new=vn, causal=True)
 
     want = call().clone()
+    torch.cuda.synchronize()
+    assert_close(want, exact, dtype)
     stream = torch.cuda.Stream()
     with torch.cuda.stream(stream):
         call()
@@ -233,6 +272,11 @@ def test_long_verify_step_appends_then_attends(D, fp8):
         k2, v2 = po.append_kv(kc, vc, bt, old, kn, vn)
         want = po.attn_f64(q, k2, v2, bt, total, 0.1, dtype, causal=True)
         kd, vd = to_dev(kc, dtype), to_dev(vc, dtype)
+    desc = pagedkv.make_desc(batch=B, num_heads=H, num_heads_k=Hk, head_dim=D, page_size=P, num_pages=kc.shape[0],
+                             block_table_stride=stride, seqlen_q=M, dtype=dtype, causal=True,
+                             kv_dtype=pagedkv.PKV_KV_DTYPE_FP8_E4M3 if fp8 else 0)
+    assert pagedkv.append_folds(desc, 0, M) is False
+    assert pagedkv.workspace_size(desc) == prefill_workspace(pagedkv.num_splits_for(desc), D)
     out = pagedkv.decode(to_dev(q, dtype), kd, vd, i32(bt), i32(old), 0.1, 0, k_new=to_dev(kn, dtype),
                          v_new=to_dev(vn, dtype), causal=True, k_scale=f32(ks), v_scale=f32(vs))
     torch.cuda.synchronize()
