@@ -984,11 +984,17 @@ hipError_t launch_d(const PartitionParams& p, hipStream_t stream, const LaunchEv
     } else {
         launch_kernel(prefill_kernel<BF16, D, false, false>, grid, block, 0, stream, part_ev, p);
     }
-    // Few streams of many parts each need the workgroups; many cut streams fill
-    // the chip as it is, and fewer workgroups are dispatched.
-    if (p.batch * p.num_heads_k * p.head_groups > kComputeUnits / 2) {
+    // Few streams of many parts each need the workgroups, and the slices from
+    // eight parts a stream on; many cut streams fill the chip as it is, and fewer
+    // workgroups are dispatched.  Measured, one slice / four (us, head_dim 128): 32
+    // streams (16 parts) 57.5 / 50.2, 128 streams (4 parts) 63.0 / 65.0.
+    const int64_t streams = static_cast<int64_t>(p.batch) * p.num_heads_k * p.head_groups;
+    if (streams > kComputeUnits / 2) {
         launch_kernel(prefill_combine_kernel<BF16, D, 16, 1>, dim3(kRows / 16, p.tile_workers), dim3(256), 0, stream,
                       comb_ev, p);
+    } else if (8 * streams > p.tile_workers) {
+        launch_kernel(prefill_combine_kernel<BF16, D, 4, 1>, dim3(kRows / 4, p.tile_workers), dim3(64), 0, stream, comb_ev,
+                      p);
     } else {
         launch_kernel(prefill_combine_kernel<BF16, D, 4, 4>, dim3(kRows / 4, p.tile_workers), dim3(256), 0, stream, comb_ev,
                       p);
