@@ -299,19 +299,21 @@ size_t workspace_bytes(const Resolved& r, const SplitPlan& plan);
 // work for the matrix cores to matter: `work` counts 32-row x 64-token blocks,
 // bounded from max_seqlen.  Measured on MI355X (bf16, append and attention,
 // prefill / decode kernels, us): head_dim 128, work 4,128 (1 row of 32 query
-// tokens over 8,192, 32/8 heads) 38.6 / 34.9, 8,256 (64 tokens) 46.7 / 51.9,
-// 16,640 52.9 / 76.5, 270,336 (8 rows of 256 tokens) 421 / 973; head_dim 64,
-// 8,256 39.9 / 38.8, 16,640 47 / 57.5; head_dim 256, 8,256 77 / 69, 10,240 81 /
-// 94, 16,640 90 / 115.  Short rows of the same work gain earlier (4,480: 8 rows
-// of 1,792 query rows 40.5 / 47.9).  With 64 query rows per KV head half of
-// each row block would be empty (work 16,512: 82-90 / 85).
+// tokens over 8,192, 32/8 heads) 33.9 / 34.5, 8,256 (64 tokens) 40.7 / 51.2,
+// 16,640 49.4 / 75.4, 270,336 (8 rows of 256 tokens) 392 / 939; head_dim 64,
+// 8,256 34.3 / 38.5, 16,640 39.5 / 56.5; head_dim 256, 8,256 64.3 / 65.4, 10,240
+// 67 / 78, 16,640 76 / 107.  One query token and 71-128 heads per KV head, 64 rows
+// of 4,096 tokens: 46-50 / 70-79.  With 64 query rows per KV head half of each
+// row block would be empty (work 16,512: 82-90 / 85).  Rows far shorter than
+// max_seqlen cost 2-8 us where a call has few streams (see the kernel's plan).
 constexpr int64_t kPrefillMinWork = 8192;
 constexpr int64_t kPrefillMinWorkD256 = 10240;
 constexpr int64_t kPrefillMinRows = 65;
 
 // Units (tiles and their streams' start) of a workgroup's share in a call that
-// does not fill the chip.  More workgroups cut the streams into more parts:
-// 1 row of 64 query tokens over 8,192 with 4 / 8 units: 63.4 / 48.2 us.
+// does not fill the chip.  More workgroups cut the streams into more parts and
+// ask for more workspace: 4 / 8 units 36.6 / 37.5 us (1 row of 64 query tokens over
+// 8,192), 37.3 / 36.8 (2 rows of 8 tokens x 16 heads), 35.0 / 39.6 (8 rows of 64 over 1,024).
 constexpr int64_t kPrefillShare = 8;
 
 // A verify step's append folds into the decode combine at no launch of its own,

@@ -131,7 +131,7 @@ constexpr int kPrefillRows = 128;
 // Row blocks of a call (batch rows x blocks) its plan holds in the LDS.
 constexpr int kPrefillEntries = 2048;
 // Units a stream is charged for its start (page ids, q, first tiles) and the
-// writing of its rows.  With 1 / 2 / 3 (and a snap of the same): 4 x 512 query
+// writing of its rows.  With 1 / 2 / 3 (and a snap of the same), in one run: 4 x 512 query
 // tokens over 0-4,096 145.7 / 140.5 / 140.9 us, 3 x 333 with a 1,024-token window
 // at head_dim 256 76.8 / 78.1 / 83.9, 2,048 tokens without a context 100 / 86 / 88.
 constexpr int kPrefillHeader = 2;

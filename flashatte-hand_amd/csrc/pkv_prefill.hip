@@ -37,8 +37,9 @@
 // query tokens, 32/8 heads, head_dim 128) 727-735 TFLOP/s counted without the
 // remainders' products, 1,090-1,100 with them, while the clock falls to about
 // 1.7 GHz; a large bf16 matrix product reaches 1,190 on the same card.  The
-// decode kernels took 1,896 us for that call, this one 767; 4 x 512 over 0-4,096 tokens
-// 306 against 142 us.  Steps on the way (4 x 512 over 0-4,096): waiting for the page
+// decode kernels took 1,892 us for that call, this one 767; 4 x 512 over 0-4,096 tokens
+// 304 against 135 (135-142 on several cards, append and merge included).  Steps on the way, each
+// in its own run (4 x 512 over 0-4,096): waiting for the page
 // ids where they were loaded 171 us, not 157; padded rows and loads through
 // registers 155; the next tile's loads in a burst and not spread over the slots
 // +15 (a load waits for the one before it at 64 bytes a clock and CU); rows
